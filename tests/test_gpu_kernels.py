@@ -339,6 +339,34 @@ def test_mfma_prefill_bytes_independent_of_grouping():
         assert torch.equal(part.view(torch.int16), whole[a:b].view(torch.int16)), (a, b)
 
 
+# Calls of 60 or more pairs per slot take the block tiles.  Slot sizes at the
+# edges of their 16-token groups, 192- and 256-token tiles (empty, one token,
+# one over a tile, several uneven tiles) with few slots (tiles of 192) and
+# with enough for every CU (tiles of 256); the shortest k loop, and a slot id
+# out of range.  Every byte equals that of the same tokens in small calls on
+# the 64-token blocks, whose outputs the oracle tests above cover.
+@pytest.mark.parametrize("H,I,reps", [(512, 256, 1), (2048, 768, 1), (2048, 768, 4),
+                                      (256, 1536, 8)])
+def test_experts_mfma_tiles_equal_the_small_blocks(H, I, reps):
+    counts = [0, 1, 15, 16, 17, 64, 191, 192, 193, 256, 257, 513] * reps
+    counts[0] += sum(counts) % 2
+    x, w, ids, w13, w2 = _counted_case(H + reps, counts, H, I)
+    xd, wd, idd, w13d, w2d = _dev_case(x, w, ids, w13, w2)
+    T, E = x.shape[0], len(counts)
+    assert 2 * T >= 60 * E
+    idd[T - 1, 1] = E + 3
+    whole = run_experts(xd, wd, idd, w13d, w2d, algo=MFMA)
+    step = 25 * E
+    for a in range(0, T, step):
+        b = min(a + step, T)
+        part = run_experts(xd[a:b].contiguous(), wd[a:b].contiguous(), idd[a:b].contiguous(),
+                           w13d, w2d, algo=MFMA)
+        assert torch.equal(part.view(torch.int16), whole[a:b].view(torch.int16)), (a, b)
+    pick = torch.arange(0, T - 1, max(1, T // 48))
+    ref = moe_forward(x[pick], w[pick], ids[pick], w13, w2, act_round="bf16")
+    assert rel_err(whole[pick.to(DEV)], ref) < 4e-3
+
+
 def test_experts_mfma_absent_slot_contributes_zero():
     x, w, ids, w13, w2 = _expert_case(6, 20, 512, 256, 8, 2, torch.bfloat16)
     slots = torch.tensor(ids, dtype=torch.int32)

@@ -8,7 +8,8 @@
 //   y[p]    = W2[s] act[p]                                        (fp32)
 //   out[t]  = bf16(sum_{k ascending} w[t,k] * y[(t, k)])
 //
-// Four launches:
+// Four launches (calls with many tokens per slot run 2 and 3 in block tiles,
+// see there):
 //   1. gather: per slot s, the ascending list of pairs routed to s and its
 //      length (block-wide ballot compaction - stable, deterministic);
 //   2. w13: block (i-panel of 64, slot s) streams the 64 gate rows and 64 up
@@ -34,6 +35,7 @@
 
 #include "common.h"
 #include "dma_pipeline.h"
+#include "tile_pipeline.h"
 
 namespace wisp {
 namespace {
@@ -66,27 +68,43 @@ struct WorkLayout {
 
 // ---------------------------------------------------------------------------
 // 1. gather: lists[s * P + j] = j-th pair (ascending) with slots[p] == s.
-// grid = nslots, block = 512 threads; each iteration covers 4096 pairs, 8
-// consecutive ones per thread, and places the matches by a block-wide
-// exclusive prefix of the per-thread counts (counts <= 8: four ballots per
-// wave for the bits, one LDS exchange across the eight waves).
+// grid = nslots; each iteration covers 8 consecutive pairs per thread and
+// places the matches by a block-wide exclusive prefix of the per-thread
+// counts (counts <= 8: four ballots per wave for the bits, one LDS exchange
+// across the waves).  What bounds a long list is the chain of iterations, so
+// the next one's pairs are loaded (16 bytes at a time where kVec) before this
+// one's are placed, one barrier an iteration suffices (two sets of totals),
+// and long lists take 16 waves instead of 8.
 // ---------------------------------------------------------------------------
 constexpr int kGatherPer = 8;
-constexpr int kGatherWaves = 8;
+constexpr int kGatherLong = 4096;  // pairs of one iteration of 8 waves
 
-__global__ __launch_bounds__(64 * kGatherWaves) void gather_kernel(
-    const int32_t* __restrict__ slots, int P, int32_t* __restrict__ lists,
-    int32_t* __restrict__ counts) {
-  __shared__ int wave_total[kGatherWaves];
+template <int NW, bool kVec>
+__global__ __launch_bounds__(64 * NW) void gather_kernel(const int32_t* __restrict__ slots, int P,
+                                                         int32_t* __restrict__ lists,
+                                                         int32_t* __restrict__ counts) {
+  __shared__ int wave_total[2][NW];
   const int s = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   int32_t* L = lists + (size_t)s * P;
   const uint64_t below = (1ull << lane) - 1ull;
-  int n = 0;  // matches before this iteration (block-uniform)
-  for (int base = 0; base < P; base += 64 * kGatherWaves * kGatherPer) {
-    const int p0 = base + tid * kGatherPer;
-    int v[kGatherPer];
+  auto load = [&](int p0, int (&v)[kGatherPer]) {
+    if (kVec && p0 + kGatherPer <= P) {
 #pragma unroll
-    for (int q = 0; q < kGatherPer; ++q) v[q] = p0 + q < P ? slots[p0 + q] : -1;
+      for (int q = 0; q < kGatherPer; q += 4) {
+        const int4 w = *reinterpret_cast<const int4*>(slots + p0 + q);
+        v[q] = w.x, v[q + 1] = w.y, v[q + 2] = w.z, v[q + 3] = w.w;
+      }
+    } else {
+#pragma unroll
+      for (int q = 0; q < kGatherPer; ++q) v[q] = p0 + q < P ? slots[p0 + q] : -1;
+    }
+  };
+  int n = 0;  // matches before this iteration (block-uniform)
+  int v[kGatherPer], next[kGatherPer];
+  load(tid * kGatherPer, v);
+  for (int base = 0, it = 0; base < P; base += 64 * NW * kGatherPer, ++it) {
+    const int p0 = base + tid * kGatherPer;
+    load(p0 + 64 * NW * kGatherPer, next);
     unsigned hit = 0;
 #pragma unroll
     for (int q = 0; q < kGatherPer; ++q) hit |= (unsigned)(v[q] == s) << q;
@@ -98,20 +116,22 @@ __global__ __launch_bounds__(64 * kGatherWaves) void gather_kernel(
       pre += __popcll(m & below) << bit;
       tot += __popcll(m) << bit;
     }
-    if (lane == 0) wave_total[wave] = tot;
-    __syncthreads();
+    if (lane == 0) wave_total[it & 1][wave] = tot;
+    // the totals of two iterations ago were read before the last barrier
+    block_lds_sync();
     int off = n, all = 0;
 #pragma unroll
-    for (int w = 0; w < kGatherWaves; ++w) {
-      off += w < wave ? wave_total[w] : 0;
-      all += wave_total[w];
+    for (int w = 0; w < NW; ++w) {
+      off += w < wave ? wave_total[it & 1][w] : 0;
+      all += wave_total[it & 1][w];
     }
-    __syncthreads();  // wave_total is rewritten by the next iteration
     int o = off + pre;
 #pragma unroll
     for (int q = 0; q < kGatherPer; ++q)
       if (hit >> q & 1u) L[o++] = p0 + q;
     n += all;
+#pragma unroll
+    for (int q = 0; q < kGatherPer; ++q) v[q] = next[q];
   }
   if (tid == 0) counts[s] = n;
 }
@@ -120,12 +140,13 @@ __global__ __launch_bounds__(64 * kGatherWaves) void gather_kernel(
 // chunk by chunk; when all blocks start at column 0, the reads in flight share
 // their low address bits and crowd a few memory channels (a pure read of the
 // Qwen3 w13 tensor in this order, non-temporal loads: 6.27 TB/s on MI355X).
-// Starting each panel at its own multiple of 64 columns, evenly spread over
-// the row, and wrapping around gives 6.99 TB/s.  The start depends only on the panel (blockIdx.x),
-// never on the slot, so an output's dot-product order is the same for any
-// slot placement or token grouping.
-__device__ inline int k_rotation(int Kdim) {
-  return (int)(blockIdx.x * (unsigned)(Kdim / 64) / gridDim.x) * 64;
+// Starting each group of panels at its own multiple of 64 columns, evenly
+// spread over the row, and wrapping around gives 6.99 TB/s.  The start depends
+// only on the output column's group (128 columns of I in w13, 256 of H in w2:
+// what the widest block covers), never on the slot, so an output's dot-product
+// order is the same for any slot placement, token grouping or block size.
+__device__ inline int k_rotation(unsigned group, unsigned groups, int Kdim) {
+  return (int)(group * (unsigned)(Kdim / 64) / groups) * 64;
 }
 
 // The w2 kernel's rotation: by the block's 256-row group of H (NG 64-row
@@ -134,8 +155,7 @@ __device__ inline int k_rotation(int Kdim) {
 template <int NG>
 __device__ inline int k_rotation_w2(int Kdim) {
   static_assert(NG == 2 || NG == 4, "64-row panels per w2 block");
-  const unsigned group = blockIdx.x * NG / 4, groups = gridDim.x * NG / 4;
-  return (int)(group * (unsigned)(Kdim / 64) / groups) * 64;
+  return k_rotation(blockIdx.x * NG / 4, gridDim.x * NG / 4, Kdim);
 }
 
 // Column of k-step offset k (0 <= k < Kdim) in a loop rotated by rot columns.
@@ -251,7 +271,7 @@ __global__ __launch_bounds__(256) void mfma_w13_dma_kernel(
     wrow[i] = reinterpret_cast<const unsigned char*>(
         W + (size_t)(r < 16 ? i0 + r : I + i0 + r - 16) * H);
   }
-  const int rot = k_rotation(H);
+  const int rot = k_rotation(blockIdx.x / 2, gridDim.x / 2, H);
   for (int m0 = 0; m0 < M; m0 += dma::kTokRows) {
     const int mrows = min(M - m0, dma::kTokRows);
     if (m0 > 0) held = dma::list_entries(list, m0, P);
@@ -310,6 +330,302 @@ __global__ __launch_bounds__(256) void mfma_w2_dma_kernel(
 #pragma unroll
         for (int g = 0; g < NG; ++g) *reinterpret_cast<f32x4*>(yr + g * 16) = acc[g][t];
       }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Large calls: the same two products in block tiles (tile_pipeline.h), 256
+// weight rows (w13: 128 gate and 128 up rows) by up to 256 or 192 tokens,
+// eight waves in persistent blocks, one per CU.  The matrix instruction and
+// the k order of every output are those of the kernels above, so the bytes
+// are too.
+// What bounds them: at the Qwen3 8192-token chunk (512 tokens a slot) w13
+// runs at 885 TFLOP/s and w2 at 637 (466 + 324 us; the 64-token blocks take
+// 1322 + 790 us).  A build without the copies takes 354 + 204 us (a plain
+// 8192^3 bf16 library product runs at 1209 TFLOP/s), one without the matrix
+// instructions 410 + 315 us: staging 64 KB a chunk and block from L2, where
+// 1 byte in 3 misses, is as long as the arithmetic and does not hide behind
+// it entirely.  Measured and not better: four 64-byte stages (512 + 371 us),
+// touching the lines three chunks ahead (557 + 361: the loads of a CU
+// return in order), 320-token tiles (492 + 335, registers spill), 128 x 128
+// tiles with two blocks per CU (545 + 351), no k rotation (447 + 329).
+// ---------------------------------------------------------------------------
+struct TileArgs {
+  const uint16_t* A;  // token matrix: x (w13) or act (w2)
+  int H, I, K, P, nslots;
+  const int32_t* lists;
+  const int32_t* counts;
+  const uint16_t* W;
+  size_t w_stride;
+  void* out;
+};
+
+template <typename Sh, bool kW13>
+struct TileLoop {
+  static constexpr int NG = Sh::NG;
+  static constexpr int kAhead = 3;  // 16-row groups a weight fragment is read ahead
+  static constexpr int kRing = kAhead + 1;
+  // groups of a chunk's second k-step left for after the next chunk's barrier
+  static constexpr int kLeft = kAhead;
+  static_assert(NG >= 4, "row groups of a wave");
+  const TileArgs& a;
+  unsigned char* smem;
+  const tile::Table* tab;
+  int N, Kdim, npanels, chunks;
+  int wave, lane, wr, wt;
+  uint32_t woff[Sh::kWCopies];
+  // this lane's place, in a stage's weight (token) rows, of the fragment of
+  // its wave's first row group (token tile) for either k-step
+  int lw[2], lt[2];
+  tile::Range tokens;
+  int q = 0;  // chunks computed so far: chunk q lies in stage q % 2
+  int j = 0;  // works taken so far
+  int stored = 0;  // token tiles a wave stored of the tile before
+
+  template <int NT>
+  struct Frags {
+    bf16x8 w[kRing], t[2][NT];
+  };
+
+  __device__ __attribute__((always_inline)) bool take(tile::Work* w) {
+    const bool found = tile::find_work(tab, tile::work_of(blockIdx.x, j++), a.nslots, npanels, w);
+    // wave-uniform by construction; the compiler sees it from here on
+    w->slot = __builtin_amdgcn_readfirstlane(w->slot);
+    w->panel = __builtin_amdgcn_readfirstlane(w->panel);
+    w->m0 = __builtin_amdgcn_readfirstlane(w->m0);
+    w->mrows = __builtin_amdgcn_readfirstlane(w->mrows);
+    return __builtin_amdgcn_readfirstlane(found);
+  }
+  __device__ __attribute__((always_inline)) int copy_row(int i) const {
+    return (i * Sh::kWaves + wave) * tile::kRowsPerCopy + lane / dma::kLanesPerRow;
+  }
+  // Weight row r of a panel, counted from the panel's first (gate) row.  w13:
+  // each wave's rows are its gate rows, then the up rows of the same columns.
+  __device__ __attribute__((always_inline)) int weight_row(int r) const {
+    constexpr int half = NG * 8;
+    if (!kW13) return r;
+    return r / (2 * half) * half + r % half + (r % (2 * half) < half ? 0 : a.I);
+  }
+  // The pairs behind this lane's token copies and the token row it touches.
+  struct Pairs {
+    int copy[Sh::kTCopies];
+  };
+  __device__ __attribute__((always_inline)) const int32_t* list(const tile::Work& w) const {
+    return a.lists + (size_t)w.slot * a.P + w.m0;
+  }
+  __device__ __attribute__((always_inline)) void pairs(const tile::Work& w, Pairs* p) const {
+    const int32_t* l = list(w);
+#pragma unroll
+    for (int i = 0; i < Sh::kTCopies; ++i) p->copy[i] = l[min(copy_row(i), w.mrows - 1)];
+  }
+  __device__ __attribute__((always_inline)) void source(const tile::Work& w, const Pairs& p,
+                                                        tile::Source<Sh>* s) const {
+    const int row0 = w.panel * (kW13 ? Sh::kRows / 2 : Sh::kRows);
+    const uint32_t rb = (uint32_t)Kdim * 2;
+    s->w = {a.W + (size_t)w.slot * a.w_stride + (size_t)row0 * Kdim, (uint32_t)(N - row0) * rb};
+#pragma unroll
+    for (int i = 0; i < Sh::kTCopies; ++i)
+      s->toff[i] = (uint32_t)(kW13 ? p.copy[i] / a.K : p.copy[i]) * rb +
+                   (((lane % dma::kLanesPerRow) ^ (copy_row(i) & 7)) << 4);
+    constexpr int per = tile::kRowsPerCopy * Sh::kWaves, step = 16 * Sh::WT;
+    s->tc = ((w.mrows + step - 1) / step * step + per - 1) / per;
+    s->rot = k_rotation(w.panel * Sh::kRows / 256, N / 256, Kdim) * 2;
+  }
+  __device__ __attribute__((always_inline)) void issue(unsigned char* stage,
+                                                       const tile::Source<Sh>& s, int c) const {
+    tile::copies<Sh>(stage, s, woff, tokens, wave, tile::chunk_byte(c, s.rot, Kdim * 2));
+  }
+  template <int NT>
+  __device__ __attribute__((always_inline)) void read_t(const unsigned char* stage, int u, int i,
+                                                        Frags<NT>& f) const {
+    f.t[u][i] = *reinterpret_cast<const bf16x8*>(
+        stage + Sh::kRows * tile::kRowBytes + lt[u] + i * Sh::WT * 16 * tile::kRowBytes);
+  }
+  // Weight fragment n of a chunk: row group n % NG of k-step n / NG.
+  template <int NT>
+  __device__ __attribute__((always_inline)) void read_w(const unsigned char* stage, int n,
+                                                        Frags<NT>& f) const {
+    f.w[n % kRing] = *reinterpret_cast<const bf16x8*>(
+        stage + lw[n / NG] + n % NG * 16 * tile::kRowBytes);
+  }
+  template <int NT>
+  __device__ __attribute__((always_inline)) void mma(int n, const Frags<NT>& f,
+                                                     f32x4 (&acc)[NG][NT]) const {
+#pragma unroll
+    for (int i = 0; i < NT; ++i)
+      acc[n % NG][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f.w[n % kRing], f.t[n / NG][i],
+                                                               acc[n % NG][i], 0, 0, 0);
+  }
+  // One chunk, from stage `rds`, with the next chunk's copies into `wrs`
+  // (distinct stages, see dma::step): fragment by fragment in the order of
+  // the matrix instructions, each read kAhead groups before its use.  The
+  // last kLeft groups of the chunk before (unless kFirst) cover the first
+  // reads, and this chunk's are left for the next call: all its fragments
+  // are then in registers, so that its stage can be overwritten.
+  template <int NT, bool kFirst>
+  __device__ __attribute__((always_inline)) void chunk(unsigned char* __restrict__ wrs,
+                                                       const unsigned char* __restrict__ rds,
+                                                       const tile::Source<Sh>& cs, int cc,
+                                                       Frags<NT>& f, f32x4 (&acc)[NG][NT]) const {
+    if (cc >= 0) issue(wrs, cs, cc);
+    __builtin_amdgcn_sched_barrier(0);
+    // positions -kLeft .. 2 NG - kLeft - 1; before position n: token
+    // fragments of the first k-step, then weight fragment n + kAhead
+#pragma unroll
+    for (int i = 0; i < NT; ++i) read_t<NT>(rds, 0, i, f);
+#pragma unroll
+    for (int n = -kLeft; n < 2 * NG - kLeft; ++n) {
+      read_w<NT>(rds, n + kAhead, f);  // its place is free: group n - 1 was its last reader
+      if (n >= 0 && n < NG - 1) {
+#pragma unroll
+        for (int i = n * NT / (NG - 1); i < (n + 1) * NT / (NG - 1); ++i)
+          read_t<NT>(rds, 1, i, f);
+      }
+      if (n >= 0)
+        mma<NT>(n, f, acc);
+      else if (!kFirst)
+        mma<NT>(2 * NG + n, f, acc);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+
+  // Waits for the next chunk (this wave's copies of it) and for every wave's
+  // reads of the one before.
+  __device__ __attribute__((always_inline)) void wait() const {
+    dma::wait_vm<0>();
+    dma::lds_barrier();
+  }
+  // The same at a tile's first chunk, whose copies are older than the stores
+  // of the tile before: those need not be waited for.  Every wave of a tile
+  // with n token tiles a wave makes exactly n * kStores of them.
+  static constexpr int kStores = kW13 ? NG / 2 : NG;
+  template <int N = Sh::NT>
+  __device__ __attribute__((always_inline)) void wait_first() const {
+    if constexpr (N > 0) {
+      if (stored != N) return wait_first<N - 1>();
+    }
+    dma::wait_vm<N * kStores>();
+    dma::lds_barrier();
+  }
+  template <int NT, bool kFirst = false>
+  __device__ __attribute__((always_inline)) void next_chunk(const tile::Source<Sh>& cs, int cc,
+                                                            Frags<NT>& f, f32x4 (&acc)[NG][NT]) {
+    chunk<NT, kFirst>(smem + (~q & 1) * Sh::kStage, smem + (q & 1) * Sh::kStage, cs, cc, f,
+                      acc);
+    ++q;
+  }
+
+  // One tile.  On entry the copies of its first chunk and the touches of the
+  // next two are issued; on return those of the next tile's are, if any.
+  template <int NT>
+  __device__ __attribute__((always_inline)) void run(tile::Work& w, tile::Source<Sh>& src,
+                                                     bool* more) {
+    f32x4 acc[NG][NT];
+#pragma unroll
+    for (int g = 0; g < NG; ++g)
+#pragma unroll
+      for (int t = 0; t < NT; ++t) acc[g][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    Frags<NT> f;
+    int pr[NT];
+    Pairs np;
+    tile::Work nw;
+    tile::Source<Sh> ns;
+    // The next tile's place and token rows are read behind the first chunk,
+    // so that they are there without a wait when its copies start.
+    wait_first();
+    const bool next = take(&nw);
+    if (next) pairs(nw, &np);
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+      pr[t] = list(w)[min((t * Sh::WT + wt) * 16 + (lane & 15), w.mrows - 1)];
+    next_chunk<NT, true>(src, 1, f, acc);
+    wait();
+    if (next) source(nw, np, &ns);
+    for (int c = 1; c < chunks - 1; ++c) {
+      next_chunk<NT>(src, c + 1, f, acc);
+      wait();
+    }
+    next_chunk<NT>(ns, next ? 0 : -1, f, acc);
+#pragma unroll
+    for (int n = 2 * NG - kLeft; n < 2 * NG; ++n) mma<NT>(n, f, acc);
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      // columns past mrows hold, and store again, the last token's values
+      if constexpr (kW13) {
+        uint16_t* ar = (uint16_t*)a.out + (size_t)pr[t] * a.I + w.panel * (Sh::kRows / 2) +
+                       wr * NG * 8 + (lane >> 4) * 4;
+#pragma unroll
+        for (int g = 0; g < NG / 2; ++g) {
+          store_act4(ar + g * 16, acc[g][t], acc[g + NG / 2][t]);
+          __builtin_amdgcn_sched_barrier(0);  // one store's temporaries at a time
+        }
+      } else {
+        float* yr = (float*)a.out + (size_t)pr[t] * a.H + w.panel * Sh::kRows + wr * NG * 16 +
+                    (lane >> 4) * 4;
+#pragma unroll
+        for (int g = 0; g < NG; ++g) *reinterpret_cast<f32x4*>(yr + g * 16) = acc[g][t];
+      }
+    }
+    stored = NT;
+    w = nw;
+    src = ns;
+    *more = next;
+  }
+};
+
+template <typename Sh, bool kW13>
+__global__ __launch_bounds__(64 * Sh::kWaves)
+__attribute__((amdgpu_waves_per_eu(Sh::kWaves / 4, Sh::kWaves / 4))) void mfma_tile_kernel(
+    TileArgs a) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char dsm[];
+  tile::Table* tab = reinterpret_cast<tile::Table*>(dsm + Sh::kTable);
+  TileLoop<Sh, kW13> L{a, dsm, tab};
+  L.N = kW13 ? 2 * a.I : a.H;
+  L.Kdim = kW13 ? a.H : a.I;
+  L.npanels = L.N / Sh::kRows;
+  L.chunks = L.Kdim * 2 / tile::kRowBytes;
+  L.wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  L.lane = threadIdx.x & 63;
+  L.wr = L.wave % Sh::WR;
+  L.wt = L.wave / Sh::WR;
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    L.lw[u] = dma::swz(L.wr * Sh::NG * 16 + (L.lane & 15), u * 4 + (L.lane >> 4));
+    L.lt[u] = dma::swz(L.wt * 16 + (L.lane & 15), u * 4 + (L.lane >> 4));
+  }
+  L.tokens = {a.A, (uint32_t)(kW13 ? a.P / a.K : a.P) * (uint32_t)(L.Kdim * 2)};
+#pragma unroll
+  for (int i = 0; i < Sh::kWCopies; ++i) {
+    const int r = L.copy_row(i);
+    L.woff[i] = (uint32_t)L.weight_row(r) * (uint32_t)(L.Kdim * 2) +
+                (((L.lane % dma::kLanesPerRow) ^ (r & 7)) << 4);
+  }
+  if (L.wave == 0) tile::fill_table(tab, a.counts, a.nslots, Sh::kToks);
+  __syncthreads();
+  tile::Work w;
+  bool more = L.take(&w);
+  if (!more) return;
+  tile::Source<Sh> src;
+  {
+    typename TileLoop<Sh, kW13>::Pairs p;
+    L.pairs(w, &p);
+    L.source(w, p, &src);
+  }
+  L.issue(dsm, src, 0);
+  while (more) {
+    const int nt = (w.mrows + 16 * Sh::WT - 1) / (16 * Sh::WT);
+    if (nt == 1)
+      L.template run<1>(w, src, &more);
+    else if (nt == 2)
+      L.template run<2>(w, src, &more);
+    else if (nt == 3)
+      L.template run<3>(w, src, &more);
+    else if (Sh::NT == 4 || nt == 4)
+      L.template run<4>(w, src, &more);
+    else if (nt == 5)
+      L.template run<(Sh::NT > 4 ? 5 : 4)>(w, src, &more);
+    else
+      L.template run<(Sh::NT > 4 ? 6 : 4)>(w, src, &more);
   }
 }
 
@@ -422,12 +738,70 @@ hipError_t launch_dma(const uint16_t* x, int H, int I, int K, int P, int nslots,
                                                       w2_stride, y, st, e2, e3);
 }
 
+constexpr int kTileBlocks = 256;  // persistent blocks: one per CU
+
+template <typename Sh, bool kW13>
+hipError_t launch_tile(const TileArgs& a, hipStream_t st, hipEvent_t e0, hipEvent_t e1) {
+  constexpr unsigned lds = Sh::kTable + sizeof(tile::Table);
+  static_assert(lds <= 160 * 1024, "LDS per block");
+  static std::atomic<uint64_t> big{0};
+  hipError_t e = allow_lds(&mfma_tile_kernel<Sh, kW13>, lds, lds, &big);
+  if (e != hipSuccess) return e;
+  launch_timed_lds(mfma_tile_kernel<Sh, kW13>, dim3(kTileBlocks), dim3(64 * Sh::kWaves), lds, st,
+                   e0, e1, a);
+  return hipSuccess;
+}
+
+// Tiles of 256 tokens, unless they would leave CUs idle (one block per CU):
+// then tiles of 192, which split the larger slots.  Measured at the Mixtral
+// 1000-token chunk's w2 (8 slots of ~250 tokens, 16 panels): 392 against
+// 341 us; at the Qwen3 8192-token chunk (128 slots of ~512, 8 panels) 324
+// against 342 us, and its w13 466 against 509 us.
+template <bool kW13>
+hipError_t launch_tiles(const TileArgs& a, hipStream_t st, hipEvent_t e0, hipEvent_t e1) {
+  using Big = tile::Shape<2, 4, 8, 4>;
+  using Small = tile::Shape<4, 2, 4, 6>;
+  const int busy = std::min(a.P, a.nslots);
+  const int64_t works = (int64_t)((kW13 ? 2 * a.I : a.H) / Big::kRows) * busy *
+                        ((a.P / busy + Big::kToks - 1) / Big::kToks);
+  return works >= kTileBlocks ? launch_tile<Big, kW13>(a, st, e0, e1)
+                              : launch_tile<Small, kW13>(a, st, e0, e1);
+}
+
+// Calls of at least this many pairs per slot take the block tiles.  The
+// 64-token blocks stream a slot's weights once per 64 of its tokens, so their
+// time steps up where slots start to need a second pass, while the tiles'
+// hardly grows with the tokens until the matrix cores bound it.  Measured,
+// 64-token blocks against tiles, w13 + w2 (us): Qwen3 48 / 64 / 96 / 128
+// pairs per slot 254 / 362 / 458 / 617 against 266 / 285 / 303 / 317;
+// Mixtral 50 / 64 / 100 / 250 508 / 728 / 981 / 2236 against
+// 665 / 692 / 738 / 881.
+constexpr int kTileMinPairs = 60;
+
+// Whether a call takes the block tiles (their 32-bit row offsets must reach
+// every byte of x, act and one expert's weights, and their buffer loads want
+// 16-byte aligned rows).
+bool tile_call(int P, int H, int I, int nslots, int T, uintptr_t addresses) {
+  const uint64_t lim = 1ull << 32;
+  return addresses % 16 == 0 && (int64_t)P >= (int64_t)kTileMinPairs * nslots && (uint64_t)T * H * 2 < lim &&
+         (uint64_t)P * I * 2 < lim && (uint64_t)I * H * 4 < lim && nslots <= kMaxExperts;
+}
+
 }  // namespace
 
 void launch_gather(const int32_t* slots, int P, int nslots, int32_t* lists, int32_t* counts,
                    hipStream_t st) {
-  hipLaunchKernelGGL(gather_kernel, dim3(nslots), dim3(64 * kGatherWaves), 0, st, slots, P, lists,
-                     counts);
+  if (P > kGatherLong) {
+    if ((uintptr_t)slots % 16 == 0)
+      hipLaunchKernelGGL((gather_kernel<16, true>), dim3(nslots), dim3(1024), 0, st, slots, P,
+                         lists, counts);
+    else
+      hipLaunchKernelGGL((gather_kernel<16, false>), dim3(nslots), dim3(1024), 0, st, slots, P,
+                         lists, counts);
+  } else {
+    hipLaunchKernelGGL((gather_kernel<8, false>), dim3(nslots), dim3(512), 0, st, slots, P, lists,
+                       counts);
+  }
 }
 
 size_t mfma_work_bytes(int T, int K, int H, int nslots) {
@@ -460,14 +834,23 @@ int experts_mfma(const void* x, int T, int H, int I, int K, const float* topk_w,
   int32_t* lists = (int32_t*)((char*)work + W.lists);
   int32_t* counts = (int32_t*)((char*)work + W.counts);
   float* y = (float*)((char*)work + W.y);
-  hipLaunchKernelGGL(gather_kernel, dim3(nslots), dim3(64 * kGatherWaves), 0, st, slots, P, lists,
-                     counts);
+  launch_gather(slots, P, nslots, lists, counts, st);
   // A slot holds a token at most once (a token's top-k experts are
   // distinct), so T bounds the rows of any slot.
   const uint16_t* xb = (const uint16_t*)x;
   const uint16_t* a13 = (const uint16_t*)w13;
   const uint16_t* a2 = (const uint16_t*)w2;
   uint16_t* ab = (uint16_t*)act;
+  if (tile_call(P, H, I, nslots, T, (uintptr_t)x | (uintptr_t)w13 | (uintptr_t)w2 |
+                                        (uintptr_t)act | w13_stride * 2 | w2_stride * 2)) {
+    const TileArgs t13{xb, H, I, K, P, nslots, lists, counts, a13, w13_stride, ab};
+    const TileArgs t2{ab, H, I, K, P, nslots, lists, counts, a2, w2_stride, y};
+    WISP_HIP_TRY((launch_tiles<true>(t13, st, ev ? ev->ev[0] : nullptr, ev ? ev->ev[1] : nullptr)));
+    WISP_HIP_TRY((launch_tiles<false>(t2, st, ev ? ev->ev[2] : nullptr, ev ? ev->ev[3] : nullptr)));
+    launch_combine(y, T, H, K, nslots, topk_w, slots, (uint16_t*)out, st);
+    WISP_HIP_TRY(hipGetLastError());
+    return WISP_OK;
+  }
   // w13 with two copy stages (three blocks per CU: 241 against 244 us at the
   // Qwen3 512-token chunk), w2 with three (its shorter rows gain nothing from
   // a third block per CU).  Measured on MI355X, these kernels also beat
