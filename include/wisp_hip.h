@@ -73,6 +73,14 @@ const char* wisp_last_error(void);
 int wisp_abi_version(void);
 /* int32 words a decision record needs for a call of T tokens x K experts. */
 int wisp_record_words(int T, int K);
+/* How a paged bf16 call of several token groups on the grouped GEMM orders
+ * its copies (host only).  record: the decided call's record; first[E]: where
+ * phase 0 finds expert e's weights (its slot before the call; -2: the slot
+ * the pager decided; -1: a later phase has it); loads: one row of four words
+ * per copy, {phase, expert, slot, 1 if that phase multiplies the expert's
+ * tokens}.  Returns the number of copies, or WISP_ERR_INVALID. */
+int wisp_plan_phases(const int32_t* record, int T, int K, int E, int cap, int32_t* first,
+                     int32_t* loads, int max_loads);
 
 /* ---- group 1: routing and the pager -------------------------------- */
 

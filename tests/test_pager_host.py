@@ -99,3 +99,53 @@ def test_host_pager_rejects_bad_ids():
     hp = HostPager(8, 4)
     rec = hp.call([[0, 9]])
     assert rec["rc"] == _lib.WISP_ERR_INVALID
+
+
+# cap from the smallest that holds a token to nearly E, calls of one token
+# group up to many, on a pager whose slots start empty and then carry over
+@pytest.mark.parametrize("E,K,cap,tmax", [(8, 2, 2, 16), (8, 2, 3, 12), (16, 2, 4, 40),
+                                           (128, 8, 8, 12), (128, 8, 24, 96), (128, 8, 64, 60),
+                                           (60, 4, 59, 80), (512, 16, 300, 90)])
+def test_phase_plan_serves_every_pair_and_leaves_the_decided_slots(hiplib, E, K, cap, tmax):
+    """Simulates the plan's copies on the slots' contents: every pair meets
+    its expert's weights in exactly one phase, the contents at the end are
+    the pager's slot table, and no plan copies more than the record."""
+    rng = np.random.default_rng(E + cap)
+    hp = HostPager(E, cap)
+    saved = 0
+    for step in range(60):
+        T = int(rng.integers(1, tmax + 1))
+        hot = rng.permutation(E)[: max(K, E // 3)] if step % 3 else np.arange(E)
+        ids = np.stack([rng.choice(hot, K, replace=False) for _ in range(T)]).astype(np.int32)
+        held = hp.s2e.copy()
+        words = hiplib.wisp_record_words(T, K)
+        rec = np.zeros(words, dtype=np.int32)
+        slots = np.zeros(T * K, dtype=np.int32)
+        assert hiplib.wisp_pager_decide_host(
+            ids.ctypes.data, T, K, E, cap, 0, hp.map.ctypes.data, hp.s2e.ctypes.data,
+            hp.tick.ctypes.data, hp.ctr.ctypes.data, slots.ctypes.data, rec.ctypes.data,
+            words) == 0
+        first = np.zeros(E, dtype=np.int32)
+        loads = np.zeros((T * K + E, 4), dtype=np.int32)
+        n = hiplib.wisp_plan_phases(rec.ctypes.data, T, K, E, cap, first.ctypes.data,
+                                    loads.ctypes.data, len(loads))
+        assert 0 <= n <= rec[6]
+        saved += int(rec[6]) - n
+        served = {}
+        for e, s in zip(ids.reshape(-1).tolist(), slots.tolist()):
+            at = s if first[e] == -2 else int(first[e])
+            if at >= 0:
+                assert held[at] == e, (step, e, at)
+                served[e] = 0
+        for phase in range(int(loads[:n, 0].max()) + 1 if n else 0):
+            rows = loads[:n][loads[:n, 0] == phase]
+            assert len(set(rows[:, 2].tolist())) == len(rows)
+            for _, e, s, use in rows.tolist():
+                held[s] = e
+                if use:
+                    assert e not in served, (step, e)
+                    served[e] = phase + 1
+        assert set(served) >= set(ids.reshape(-1).tolist()), step
+        full = hp.s2e >= 0
+        assert np.array_equal(held[full], hp.s2e[full]), step
+    assert saved > 0 or cap == E - 1

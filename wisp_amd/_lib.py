@@ -82,6 +82,7 @@ SIGNATURES = {
     "wisp_pack_bf16_stride": (_sz, [_i32, _i32, _i32, _vp, _sz, _vp, _sz]),
     "wisp_pack_bf16": (_i32, [_i32, _i32, _i32, _vp, _sz, _vp, _sz, _vp, _sz]),
     "wisp_record_words": (_i32, [_i32, _i32]),
+    "wisp_plan_phases": (_i32, [_vp, _i32, _i32, _i32, _i32, _vp, _vp, _i32]),
     "wisp_route_topk_softmax": (_i32, [_vp, _i32, _i32, _i32, _i32, _i32, _vp, _vp, _vp, _vp]),
     "wisp_pager_decide": (_i32, [_vp, _i32, _i32, _i32, _i32, _i32, _vp, _vp, _vp, _vp, _vp,
                                  _vp, _i32, _vp]),

@@ -143,6 +143,14 @@ struct StageEvents {
   hipEvent_t ev[4];
 };
 
+// Where a phase of a paged call finds its experts' weights: the slot of each
+// expert it covers, kDecided for the pager's own slots[p], kNone otherwise.
+// A kernel argument.
+struct PhaseTable {
+  static constexpr int16_t kNone = -1, kDecided = -2;
+  int16_t slot[kMaxExperts];
+};
+
 // Per slot s < nslots, the ascending list of the pairs p < P with
 // slots[p] == s (lists[s * P + j]) and its length (counts[s]); one wave per
 // slot, ballot compaction (deterministic).  Defined with the bf16 grouped

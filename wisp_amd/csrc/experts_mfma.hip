@@ -781,9 +781,9 @@ constexpr int kTileMinPairs = 60;
 // Whether a call takes the block tiles (their 32-bit row offsets must reach
 // every byte of x, act and one expert's weights, and their buffer loads want
 // 16-byte aligned rows).
-bool tile_call(int P, int H, int I, int nslots, int T, uintptr_t addresses) {
+bool tile_call(int P, int H, int I, int nslots, int spread, int T, uintptr_t addresses) {
   const uint64_t lim = 1ull << 32;
-  return addresses % 16 == 0 && (int64_t)P >= (int64_t)kTileMinPairs * nslots && (uint64_t)T * H * 2 < lim &&
+  return addresses % 16 == 0 && (int64_t)P >= (int64_t)kTileMinPairs * spread && (uint64_t)T * H * 2 < lim &&
          (uint64_t)P * I * 2 < lim && (uint64_t)I * H * 4 < lim && nslots <= kMaxExperts;
 }
 
@@ -804,6 +804,9 @@ void launch_gather(const int32_t* slots, int P, int nslots, int32_t* lists, int3
   }
 }
 
+int experts_mfma_combine(int T, int H, int K, const float* topk_w, const int32_t* slots,
+                         int nslots, const void* work, void* out, hipStream_t st);
+
 size_t mfma_work_bytes(int T, int K, int H, int nslots) {
   if (T < 1 || K < 1 || H < 1 || nslots < 1) return 0;
   return WorkLayout(T * K, H, nslots).total;
@@ -814,11 +817,15 @@ bool mfma_supported(int H, int I) {
   return H >= kKAlign && I >= kKAlign && H % kKAlign == 0 && I % kKAlign == 0;
 }
 
-int experts_mfma(const void* x, int T, int H, int I, int K, const float* topk_w,
-                 const int32_t* slots, int nslots, const void* w13, size_t w13_stride,
-                 const void* w2, size_t w2_stride, void* act, void* out, void* work,
-                 size_t work_bytes, hipStream_t st, const StageEvents* ev) {
-  if (T == 0) return WISP_OK;
+namespace {
+
+// The pair lists, w13 and w2 of a call's pairs with a slot in [0, nslots):
+// their fp32 rows of y in the work buffer.  `spread`: the number of experts
+// the call's pairs spread over, for the choice of kernels.
+int mfma_pairs(const void* x, int T, int H, int I, int K, const int32_t* slots, int nslots,
+               const void* w13, size_t w13_stride, const void* w2, size_t w2_stride, void* act,
+               void* work, size_t work_bytes, int spread, hipStream_t st,
+               const StageEvents* ev) {
   if (!mfma_supported(H, I)) {
     wisp_set_last_error("MFMA path needs hidden and intermediate sizes that are multiples of 256",
                         "MFMA experts");
@@ -841,24 +848,70 @@ int experts_mfma(const void* x, int T, int H, int I, int K, const float* topk_w,
   const uint16_t* a13 = (const uint16_t*)w13;
   const uint16_t* a2 = (const uint16_t*)w2;
   uint16_t* ab = (uint16_t*)act;
-  if (tile_call(P, H, I, nslots, T, (uintptr_t)x | (uintptr_t)w13 | (uintptr_t)w2 |
-                                        (uintptr_t)act | w13_stride * 2 | w2_stride * 2)) {
+  if (tile_call(P, H, I, nslots, spread, T, (uintptr_t)x | (uintptr_t)w13 | (uintptr_t)w2 |
+                                                (uintptr_t)act | w13_stride * 2 |
+                                                w2_stride * 2)) {
     const TileArgs t13{xb, H, I, K, P, nslots, lists, counts, a13, w13_stride, ab};
     const TileArgs t2{ab, H, I, K, P, nslots, lists, counts, a2, w2_stride, y};
     WISP_HIP_TRY((launch_tiles<true>(t13, st, ev ? ev->ev[0] : nullptr, ev ? ev->ev[1] : nullptr)));
     WISP_HIP_TRY((launch_tiles<false>(t2, st, ev ? ev->ev[2] : nullptr, ev ? ev->ev[3] : nullptr)));
-    launch_combine(y, T, H, K, nslots, topk_w, slots, (uint16_t*)out, st);
-    WISP_HIP_TRY(hipGetLastError());
-    return WISP_OK;
+  } else {
+    // w13 with two copy stages (three blocks per CU: 241 against 244 us at the
+    // Qwen3 512-token chunk), w2 with three (its shorter rows gain nothing from
+    // a third block per CU).  Measured on MI355X, these kernels also beat
+    // register-streaming ones at every call size, down to 4 tokens (71 against
+    // 109 us at the Qwen3 shape).
+    WISP_HIP_TRY((launch_dma<2>(xb, H, I, K, P, nslots, lists, counts, a13, w13_stride, a2,
+                                w2_stride, ab, y, st, ev)));
   }
-  // w13 with two copy stages (three blocks per CU: 241 against 244 us at the
-  // Qwen3 512-token chunk), w2 with three (its shorter rows gain nothing from
-  // a third block per CU).  Measured on MI355X, these kernels also beat
-  // register-streaming ones at every call size, down to 4 tokens (71 against
-  // 109 us at the Qwen3 shape).
-  WISP_HIP_TRY((launch_dma<2>(xb, H, I, K, P, nslots, lists, counts, a13, w13_stride, a2,
-                              w2_stride, ab, y, st, ev)));
-  launch_combine(y, T, H, K, nslots, topk_w, slots, (uint16_t*)out, st);
+  WISP_HIP_TRY(hipGetLastError());
+  return WISP_OK;
+}
+
+// slots[p] of one phase (see experts_mfma_phase).
+__global__ __launch_bounds__(256) void phase_slots_kernel(const int32_t* __restrict__ ids,
+                                                          const int32_t* __restrict__ slots,
+                                                          int P, PhaseTable t,
+                                                          int32_t* __restrict__ out) {
+  const int p = blockIdx.x * 256 + threadIdx.x;
+  if (p >= P) return;
+  const int e = ids[p];
+  const int s = e >= 0 && e < kMaxExperts ? t.slot[e] : PhaseTable::kNone;
+  out[p] = s == PhaseTable::kDecided ? slots[p] : s;
+}
+
+}  // namespace
+
+int experts_mfma(const void* x, int T, int H, int I, int K, const float* topk_w,
+                 const int32_t* slots, int nslots, const void* w13, size_t w13_stride,
+                 const void* w2, size_t w2_stride, void* act, void* out, void* work,
+                 size_t work_bytes, hipStream_t st, const StageEvents* ev) {
+  if (T == 0) return WISP_OK;
+  const int rc = mfma_pairs(x, T, H, I, K, slots, nslots, w13, w13_stride, w2, w2_stride, act,
+                            work, work_bytes, nslots, st, ev);
+  if (rc != WISP_OK) return rc;
+  return experts_mfma_combine(T, H, K, topk_w, slots, nslots, work, out, st);
+}
+
+// The pairs of the experts that a phase of a paged call covers: their y rows
+// in the work buffer.  phase_slots: P ints of scratch.
+int experts_mfma_phase(const void* x, int T, int H, int I, int K, const int32_t* ids,
+                       const int32_t* slots, const PhaseTable& t, int32_t* phase_slots,
+                       int nslots, int num_experts, const void* w13, size_t w13_stride,
+                       const void* w2, size_t w2_stride, void* act, void* work,
+                       size_t work_bytes, hipStream_t st, const StageEvents* ev) {
+  hipLaunchKernelGGL(phase_slots_kernel, dim3((T * K + 255) / 256), dim3(256), 0, st, ids, slots,
+                     T * K, t, phase_slots);
+  return mfma_pairs(x, T, H, I, K, phase_slots, nslots, w13, w13_stride, w2, w2_stride, act, work,
+                    work_bytes, num_experts, st, ev);
+}
+
+// out from the y rows of every pair with a slot.
+int experts_mfma_combine(int T, int H, int K, const float* topk_w, const int32_t* slots,
+                         int nslots, const void* work, void* out, hipStream_t st) {
+  const WorkLayout W(T * K, H, nslots);
+  launch_combine((const float*)((const char*)work + W.y), T, H, K, nslots, topk_w, slots,
+                 (uint16_t*)out, st);
   WISP_HIP_TRY(hipGetLastError());
   return WISP_OK;
 }

@@ -54,6 +54,14 @@ struct PageInArgs {
 
 int launch_pagein(const PageInArgs& a, hipStream_t st, hipEvent_t ev_start, hipEvent_t ev_stop);
 
+// (expert, slot) pairs chosen on the host, as a kernel argument; a.loads and
+// a.count are not used, a.n is their number.
+struct PageInList {
+  int16_t pair[kMaxExperts][2];
+};
+int launch_pagein_list(const PageInArgs& a, const PageInList& list, hipStream_t st,
+                       hipEvent_t ev_start, hipEvent_t ev_stop);
+
 // The pager wave's arguments in a fused one-token decode launch (page-in,
 // w13 and the pager in one grid; the layer's call with top-k == cap).
 struct DecodePagerArgs {

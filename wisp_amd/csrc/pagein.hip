@@ -17,25 +17,35 @@
 namespace wisp {
 namespace {
 
-__global__ __launch_bounds__(256) void pagein_kernel(PageInArgs a) {
-  const int n = a.count ? *a.count : a.n;
+__device__ inline void page_in_one(const PageInArgs& a, int e, int s) {
+  if (e < 0 || e >= a.num_experts || s < 0 || s >= a.cap) return;
+  if (a.pk.m) {
+    unpack_expert(a.pk, e, s, blockIdx.x, gridDim.x);
+    return;
+  }
+  for (int q = 0; q < a.nplanes; ++q) {
+    const PageInPlane& pl = a.p[q];
+    copy_range(pl.m + (size_t)e * pl.m_stride, pl.d + (size_t)s * pl.d_stride, pl.bytes,
+               blockIdx.x, gridDim.x);
+  }
+}
+
+__device__ inline void tell_count(const PageInArgs& a, int n) {
   if (a.hist && blockIdx.x == 0 && threadIdx.x == 0) {
     *a.hist = n;
     __threadfence_system();
   }
-  for (int j = 0; j < n; ++j) {
-    const int e = a.loads[2 * j], s = a.loads[2 * j + 1];
-    if (e < 0 || e >= a.num_experts || s < 0 || s >= a.cap) continue;
-    if (a.pk.m) {
-      unpack_expert(a.pk, e, s, blockIdx.x, gridDim.x);
-      continue;
-    }
-    for (int q = 0; q < a.nplanes; ++q) {
-      const PageInPlane& pl = a.p[q];
-      copy_range(pl.m + (size_t)e * pl.m_stride, pl.d + (size_t)s * pl.d_stride, pl.bytes,
-                 blockIdx.x, gridDim.x);
-    }
-  }
+}
+
+__global__ __launch_bounds__(256) void pagein_kernel(PageInArgs a) {
+  const int n = a.count ? *a.count : a.n;
+  tell_count(a, n);
+  for (int j = 0; j < n; ++j) page_in_one(a, a.loads[2 * j], a.loads[2 * j + 1]);
+}
+
+__global__ __launch_bounds__(256) void pagein_list_kernel(PageInArgs a, PageInList list) {
+  tell_count(a, a.n);
+  for (int j = 0; j < a.n; ++j) page_in_one(a, list.pair[j][0], list.pair[j][1]);
 }
 
 }  // namespace
@@ -44,6 +54,14 @@ int launch_pagein(const PageInArgs& a, hipStream_t st, hipEvent_t ev_start, hipE
   // packed masters: twice the blocks, since a chunk's loads move fewer bytes
   launch_timed(pagein_kernel, dim3(a.pk.m ? 2 * kPageInBlocks : kPageInBlocks), dim3(256), st,
                ev_start, ev_stop, a);
+  WISP_HIP_TRY(hipGetLastError());
+  return WISP_OK;
+}
+
+int launch_pagein_list(const PageInArgs& a, const PageInList& list, hipStream_t st,
+                       hipEvent_t ev_start, hipEvent_t ev_stop) {
+  launch_timed(pagein_list_kernel, dim3(a.pk.m ? 2 * kPageInBlocks : kPageInBlocks), dim3(256),
+               st, ev_start, ev_stop, a, list);
   WISP_HIP_TRY(hipGetLastError());
   return WISP_OK;
 }
