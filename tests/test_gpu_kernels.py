@@ -163,6 +163,46 @@ def test_gpu_pager_above_the_staged_id_limit(E, K, cap, T):
                                        ora.stats_evict, ora.stats_hits], step
 
 
+# More than 4096 pairs read by the whole block: a count that no quad or pass
+# of ids divides, more than one pass (8192 pairs), ids at an address that is
+# not 16-byte aligned, all experts in one group, the widest masks.
+@pytest.mark.parametrize("E,K,cap,T,shift", [(127, 3, 127, 1367, 0), (128, 8, 128, 4099, 0),
+                                             (128, 8, 128, 600, 1), (512, 5, 512, 3001, 3)])
+def test_gpu_pager_wide_calls_of_one_group(E, K, cap, T, shift):
+    rng = np.random.default_rng(E + T)
+    ora, dp = PagerOracle(E, cap), DevPager(E, cap)
+    hold = torch.zeros(T * K + 4, dtype=torch.int32, device=DEV)
+    words = _lib.lib().wisp_record_words(T, K)
+    for step in range(2):
+        live = rng.permutation(E)[: E - 5 + 5 * step]  # the second call loads five more
+        ids = np.stack([rng.choice(live, K, replace=False) for _ in range(T)]).astype(np.int32)
+        hold[shift:shift + T * K] = torch.from_numpy(ids.reshape(-1)).to(DEV)
+        rec = torch.zeros(words, dtype=torch.int32, pin_memory=True)
+        slots = torch.full((T * K,), -7, dtype=torch.int32, device=DEV)
+
+        def call():
+            return _lib.lib().wisp_pager_decide(
+                hold.data_ptr() + 4 * shift, T, K, E, cap, 0, dp.map.data_ptr(),
+                dp.s2e.data_ptr(), dp.tick.data_ptr(), dp.ctr.data_ptr(), slots.data_ptr(),
+                rec.data_ptr(), words, _lib.stream_handle())
+
+        # an id out of range is refused and leaves the state alone
+        before = dp.s2e.tolist()
+        hold[shift + T * K - 1] = E
+        assert call() == 0
+        torch.cuda.synchronize()
+        assert rec[0] == _lib.WISP_ERR_INVALID and dp.s2e.tolist() == before
+        assert slots.unique().tolist() == [-1]
+        hold[shift + T * K - 1] = int(ids[-1, -1])
+        assert call() == 0
+        torch.cuda.synchronize()
+        res = ora.forward(ids.tolist())
+        oracle_trace_matches(res, parse_record(rec.numpy(), T, K))
+        assert slots.view(T, K).tolist() == res["slots"]
+        assert dp.s2e.tolist() == ora.slot_to_expert and dp.tick.tolist() == ora.lru_tick
+        assert dp.map.tolist() == ora.expert_map()
+
+
 def test_gpu_pager_overflow():
     dp = DevPager(8, 2)
     rec = dp.call([[0, 1, 1], [2, 3, 4]], 3)

@@ -203,6 +203,100 @@ __global__ __launch_bounds__(64) void pager_kernel(
       ctr_g, slots_g, flags_g, loads_g, rec, rec_host, sm, fr);
 }
 
+// A call with more ids than the pager's LDS holds: the pager wave read them
+// from global memory three times over (to check them, to find their union, to
+// write their slots), 146 us at 32768 ids, most of it waiting; 23 us so.  The
+// block's eight waves read them once before it, four a lane and four loads in
+// flight, and write the slots of a one-group call after it.
+constexpr int kWideThreads = 512;
+
+template <int VALS>
+__global__ __launch_bounds__(kWideThreads) void pager_wide_kernel(
+    const int32_t* __restrict__ ids, int T, int K, int E, int cap, int single_group,
+    int32_t* __restrict__ map_g, int32_t* __restrict__ s2e_g, int64_t* __restrict__ tick_g,
+    int64_t* __restrict__ ctr_g, int32_t* __restrict__ slots_g, int32_t* __restrict__ flags_g,
+    int32_t* __restrict__ loads_g, int32_t* __restrict__ rec, int32_t* __restrict__ rec_host) {
+  __shared__ PagerSmemT<kMaxExperts> sm;
+  __shared__ FusedRouteSmemT<1> fr;
+  __shared__ WideCall wide;
+  __shared__ int32_t present[64 * VALS];
+  const int tid = threadIdx.x, P = T * K;
+  const bool quads = (uintptr_t)ids % 16 == 0;
+  // four consecutive ids from p on (-1 past the call's)
+  auto load4 = [&](int p) -> int4 {
+    if (quads && p + 3 < P) return *reinterpret_cast<const int4*>(ids + p);
+    return make_int4(p < P ? ids[p] : -1, p + 1 < P ? ids[p + 1] : -1,
+                     p + 2 < P ? ids[p + 2] : -1, p + 3 < P ? ids[p + 3] : -1);
+  };
+  constexpr int kAtOnce = 4, kStep = 4 * kWideThreads;
+  for (int e = tid; e < 64 * VALS; e += kWideThreads) present[e] = 0;
+  if (tid == 0) wide.bad = wide.write = 0;
+  __syncthreads();
+  bool bad = false;
+  for (int p0 = 4 * tid; p0 < P; p0 += kAtOnce * kStep) {
+    int4 v[kAtOnce];
+#pragma unroll
+    for (int u = 0; u < kAtOnce; ++u) v[u] = load4(p0 + u * kStep);
+#pragma unroll
+    for (int u = 0; u < kAtOnce; ++u) {
+      const int e[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        if (p0 + u * kStep + i >= P) continue;
+        if ((unsigned)e[i] < (unsigned)E)
+          present[e[i]] = 1;
+        else
+          bad = true;
+      }
+    }
+  }
+  if (bad) wide.bad = 1;
+  __syncthreads();
+  for (int v = tid >> 6; v < VALS; v += kWideThreads / 64) {
+    const uint64_t b = __ballot(present[v * 64 + (tid & 63)] != 0);
+    if ((tid & 63) == 0) {
+      wide.all[2 * v] = (uint32_t)b;
+      wide.all[2 * v + 1] = (uint32_t)(b >> 32);
+    }
+  }
+  __syncthreads();
+  if (tid < 64)
+    pager_wave<float, VALS, false, kMaxExperts, 1>(
+        ids, nullptr, 0, nullptr, nullptr, T, K, E, cap, single_group, map_g, s2e_g, tick_g,
+        ctr_g, slots_g, flags_g, loads_g, rec, rec_host, sm, fr, &wide);
+  __syncthreads();
+  if (!wide.write) return;
+  for (int p0 = 4 * tid; p0 < P; p0 += kAtOnce * kStep) {
+    int4 v[kAtOnce];
+#pragma unroll
+    for (int u = 0; u < kAtOnce; ++u) v[u] = load4(p0 + u * kStep);
+#pragma unroll
+    for (int u = 0; u < kAtOnce; ++u) {
+      const int p = p0 + u * kStep;
+      const int e[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
+      int32_t m[4], f[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int x = p + i < P ? e[i] : 0;
+        m[i] = sm.map[x];
+        f[i] = pair_word(m[i], (sm.loaded[x >> 5] >> (x & 31)) & 1u ? x : -1);
+      }
+      if (p + 3 < P) {
+        if (slots_g) *reinterpret_cast<Words4*>(slots_g + p) = Words4{m[0], m[1], m[2], m[3]};
+        if (flags_g)
+          *reinterpret_cast<Words4*>(flags_g + 1 + p) = Words4{f[0], f[1], f[2], f[3]};
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (p + i < P) {
+            if (slots_g) slots_g[p + i] = m[i];
+            if (flags_g) flags_g[1 + p + i] = f[i];
+          }
+      }
+    }
+  }
+}
+
 }  // namespace
 
 int launch_pager(const int32_t* ids, const void* logits, int logits_dtype, int renorm,
@@ -271,9 +365,9 @@ int launch_pager(const int32_t* ids, const void* logits, int logits_dtype, int r
                          single_group, map, s2e, tick, ctr, slots, flags, loads, rec,
                          rec_host);
     else
-      hipLaunchKernelGGL((pager_kernel<float, V, false, false>), dim3(1), dim3(64), 0, stream,
-                         ids, nullptr, renorm, topk_w, topk_ids, T, K, E, cap, single_group, map,
-                         s2e, tick, ctr, slots, flags, loads, rec, rec_host);
+      hipLaunchKernelGGL((pager_wide_kernel<V>), dim3(1), dim3(kWideThreads), 0, stream, ids, T, K,
+                         E, cap, single_group, map, s2e, tick, ctr, slots, flags, loads, rec,
+                         rec_host);
   });
   WISP_HIP_TRY(hipGetLastError());
   return WISP_OK;

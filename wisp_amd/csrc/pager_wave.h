@@ -100,6 +100,16 @@ __device__ inline int set_table_size(int n) {
 // REGS (decided at launch): a call whose ids were routed before the launch,
 // on the register path - batched decode and prefill chunks - compiled
 // without the routing and the LDS path.
+// What the other waves of the pager's block do for a call whose ids do not
+// fit its LDS: before pager_wave they have read the ids (`bad`: one lies
+// outside [0, E); `all`: the experts they name), and after it they write the
+// slot and flag words of a call that is one group (`write`, set by
+// pager_wave).
+struct WideCall {
+  uint32_t all[kMaxExperts / 32];
+  int bad, write;
+};
+
 template <typename TL, int VALS, bool STAGED, int MAXE, int MAXP, bool ONE = false,
           bool REGS = false>
 __device__ __attribute__((always_inline)) inline void pager_wave(
@@ -108,7 +118,8 @@ __device__ __attribute__((always_inline)) inline void pager_wave(
     int single_group, int32_t* __restrict__ map_g, int32_t* __restrict__ s2e_g,
     int64_t* __restrict__ tick_g, int64_t* __restrict__ ctr_g, int32_t* __restrict__ slots_g,
     int32_t* __restrict__ flags_g, int32_t* __restrict__ loads_g, int32_t* __restrict__ rec,
-    int32_t* __restrict__ rec_host, PagerSmemT<MAXE>& sm, FusedRouteSmemT<MAXP>& fr) {
+    int32_t* __restrict__ rec_host, PagerSmemT<MAXE>& sm, FusedRouteSmemT<MAXP>& fr,
+    WideCall* wide = nullptr) {
   static_assert(!ONE || (VALS == 2 && STAGED), "a routed one-token call on the register path");
   static_assert(!REGS || (VALS == 2 && !ONE), "ids given, on the register path");
   if constexpr (ONE) T = 1;
@@ -307,7 +318,9 @@ __device__ __attribute__((always_inline)) inline void pager_wave(
   int done_p = 0;
 
   // Validate the ids not checked above, four a lane at a time.
-  if (!routed && !kCheckStaged)
+  if (wide)
+    bad = wide->bad != 0;
+  else if (!routed && !kCheckStaged)
     for (int p0 = 0; p0 < P; p0 += 256) {
       int e[4];
 #pragma unroll
@@ -480,7 +493,11 @@ __device__ __attribute__((always_inline)) inline void pager_wave(
           uint32_t all[W];
 #pragma unroll
           for (int w = 0; w < W; ++w) all[w] = 0u;
-          if (STAGED && (P & 3) == 0) {
+          if (wide) {
+#pragma unroll
+            for (int w = 0; w < W; ++w)
+              all[w] = (uint32_t)__builtin_amdgcn_readfirstlane((int)wide->all[w]);
+          } else if (STAGED && (P & 3) == 0) {
             // a presence word per expert (sm.cand, free until the evictions
             // fill it), set by every pair's id (validated above), four
             // consecutive ids a lane by one 16-byte LDS read (a lane past
@@ -1025,7 +1042,9 @@ __device__ __attribute__((always_inline)) inline void pager_wave(
       // with K a multiple of 4 a quad never straddles the group's end; a
       // lane past it re-reads the group's first quad and stores nothing
       const bool quads = STAGED && (K & 3) == 0;
-      for (int p0 = t0 * K; p0 < p1; p0 += 512) {
+      const bool later = wide && t0 == 0 && t1 == T;  // by the whole block
+      if (later && lane == 0) wide->write = 1;
+      for (int p0 = later ? p1 : t0 * K; p0 < p1; p0 += 512) {
         int e[8], m[8], f[8];
         uint32_t ld[8];
 #pragma unroll
