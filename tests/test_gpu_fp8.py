@@ -245,6 +245,33 @@ def test_experts_fp8_grouped_bytes_equal_across_kernel_families(H, I, block):
     assert _rel(full_act, want_act) < REL_TOL and _rel(full, want) < REL_TOL
 
 
+# Calls of 60 or more pairs per slot take the block tiles.  Slot sizes at the
+# edges of their 16-token groups and 256-token tiles, the shortest k loop, a
+# scale block of 64 rows, a slot id out of range; (8, ...): more tiles than
+# persistent blocks.  Every byte equals that of small calls on the 64-token
+# blocks, which the oracle tests above cover.
+@pytest.mark.parametrize("H,I,block,reps", [(512, 256, (64, 128), 1), (256, 384, (128, 128), 1),
+                                            (1024, 768, (128, 128), 8)])
+def test_experts_fp8_tiles_equal_the_small_blocks(H, I, block, reps):
+    counts = np.array([0, 1, 15, 16, 17, 64, 255, 256, 257, 513] * reps)
+    counts[0] += counts.sum() % 2
+    E, T = len(counts), int(counts.sum()) // 2
+    labels = np.repeat(np.arange(E), counts).astype(np.int32)
+    ids = np.stack([labels[:T], labels[T:]], axis=1)
+    ids[T - 1, 1] = E + 3
+    _, w13, w2, s13, s2 = _experts(E, H, I, block, seed=31)
+    tw = np.random.default_rng(32).uniform(0.05, 1.0, (T, 2)).astype(np.float32)
+    x = torch.randn((T, H), generator=torch.Generator().manual_seed(33)).to(torch.bfloat16)
+    mfma = _lib.WISP_ALGO_MFMA
+    assert 2 * T >= 60 * E
+    full, _ = _run_experts(x, ids, tw, w13, w2, s13, s2, block, algo=mfma)
+    step = 25 * E
+    for a in range(0, T, step):
+        part, _ = _run_experts(x[a:a + step], ids[a:a + step], tw[a:a + step], w13, w2, s13, s2,
+                               block, algo=mfma)
+        assert torch.equal(part.view(torch.int32), full[a:a + step].view(torch.int32)), a
+
+
 def test_experts_fp8_decode_kernels_over_256_pairs():
     """The decode kernels' in-memory slot scan (launches of more than 256
     pairs) against the oracle."""

@@ -42,6 +42,7 @@
 
 #include "common.h"
 #include "dma_pipeline.h"
+#include "tile_pipeline.h"
 #include "pagein.h"
 #include "pager_core.h"
 
@@ -1556,24 +1557,357 @@ __global__ __launch_bounds__(256) void fp8_w2_dma_kernel(
   }
 }
 
+// ---------------------------------------------------------------------------
+// Large calls: both products in block tiles (tile_pipeline.h), 256 weight
+// rows (w13: 128 gate and 128 up rows) by up to Sh::kToks tokens, persistent
+// blocks of eight waves, one per CU; a chunk is one 128-column k-block.  The
+// steps of an output are those of the kernels above, so the bytes are too.
+// What bounds them: at the Qwen3-FP8 4096-token chunk (256 tokens a slot)
+// 292 + 155 us (w13 + w2; the 64-token blocks 389 + 236 us), at 8192 tokens
+// 451 + 255 us (750 + 447).  Per product the operation's separate roundings
+// take 12 vector instructions, 1.5 times the matrix instruction's own time;
+// a build without the copies takes 228 + 118 us, one without the matrix
+// instructions 190 + 125 us.  Measured and not better: issuing the next row
+// group's products before scaling this one's (302 + 156 us, registers spill),
+// 128 rows by 256 tokens (310 + 192), 256 by 128 tokens (290 + 165; 486 + 294
+// at 8192 tokens), sixteen waves (380 + 259, spills).
+// ---------------------------------------------------------------------------
+struct Fp8TileArgs {
+  const uint8_t* A;      // codes: xq [T][H] (w13) or aq [P][I] (w2)
+  const float* scales;   // their scales [rows][Kdim / 128]
+  int H, I, K, P, rows, nslots;
+  const int32_t* lists;
+  const int32_t* counts;
+  const float* topk_w;
+  const uint8_t* W;
+  size_t w_stride;
+  const float* wscale;
+  size_t ws_stride;
+  int block_n;
+  uint16_t* out;         // act [P][I] or y [P][H]
+};
+
+template <typename Sh, bool kW13>
+struct Fp8TileLoop {
+  static constexpr int NG = Sh::NG, NT = Sh::NT;
+  static constexpr int kStores = kW13 ? NG / 2 : NG;  // per token tile
+  const Fp8TileArgs& a;
+  unsigned char* smem;
+  const tile::Table* tab;
+  int N, Kdim, npanels, chunks;
+  int wave, lane, wr, wt;
+  uint32_t woff, wstep[Sh::kWCopies];
+  // this lane's place, in a stage's weight (token) rows, of the two halves of
+  // the operand of its wave's first row group (token tile)
+  int lw[2], lt[2];
+  tile::Range tokens;
+  int q = 0;       // chunks computed so far: chunk q lies in stage q % 2
+  int j = 0;       // works taken so far
+  int stored = 0;  // token tiles a wave stored of the tile before
+  float sx[NT];    // the token scales of the chunk computed next
+
+  // The pairs behind this lane's token copies and output columns, and (by
+  // place_scales()) where the columns' scales are.
+  struct Pairs {
+    int copy[Sh::kTCopies], out[NT];
+    uint32_t scale[NT];
+  };
+  __device__ __attribute__((always_inline)) bool take(tile::Work* w) {
+    const bool found = tile::find_work(tab, tile::work_of(blockIdx.x, j++), a.nslots, npanels, w);
+    // wave-uniform by construction; the compiler sees it from here on
+    w->slot = __builtin_amdgcn_readfirstlane(w->slot);
+    w->panel = __builtin_amdgcn_readfirstlane(w->panel);
+    w->m0 = __builtin_amdgcn_readfirstlane(w->m0);
+    w->mrows = __builtin_amdgcn_readfirstlane(w->mrows);
+    return __builtin_amdgcn_readfirstlane(found);
+  }
+  __device__ __attribute__((always_inline)) int copy_row(int i) const {
+    return (i * Sh::kWaves + wave) * tile::kRowsPerCopy + lane / dma::kLanesPerRow;
+  }
+  // Weight row r of a panel, counted from the panel's first (gate) row.  w13:
+  // each wave's rows are its gate rows, then the up rows of the same columns.
+  __device__ __attribute__((always_inline)) int weight_row(int r) const {
+    constexpr int half = NG * 8;
+    if (!kW13) return r;
+    return r / (2 * half) * half + r % half + (r % (2 * half) < half ? 0 : a.I);
+  }
+  __device__ __attribute__((always_inline)) void pairs(const tile::Work& w, Pairs* p) const {
+    const int32_t* l = a.lists + (size_t)w.slot * a.P + w.m0;
+#pragma unroll
+    for (int i = 0; i < Sh::kTCopies; ++i) p->copy[i] = l[min(copy_row(i), w.mrows - 1)];
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+      p->out[t] = l[min((t * Sh::WT + wt) * 16 + (lane & 15), w.mrows - 1)];
+  }
+  __device__ __attribute__((always_inline)) int panel_row(const tile::Work& w) const {
+    return w.panel * (kW13 ? Sh::kRows / 2 : Sh::kRows);
+  }
+  __device__ __attribute__((always_inline)) void place_scales(Pairs& p) const {
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+      p.scale[t] = (uint32_t)(kW13 ? p.out[t] / a.K : p.out[t]) * (uint32_t)chunks;
+  }
+  __device__ __attribute__((always_inline)) void source(const tile::Work& w, const Pairs& p,
+                                                        tile::Source<Sh>* s) const {
+    const int row0 = panel_row(w);
+    s->w = {a.W + (size_t)w.slot * a.w_stride + (size_t)row0 * Kdim,
+            (uint32_t)(N - row0) * (uint32_t)Kdim};
+#pragma unroll
+    for (int i = 0; i < Sh::kTCopies; ++i)
+      s->toff[i] = (uint32_t)(kW13 ? p.copy[i] / a.K : p.copy[i]) * (uint32_t)Kdim +
+                   (((lane % dma::kLanesPerRow) ^ (copy_row(i) & 7)) << 4);
+    constexpr int per = tile::kRowsPerCopy * Sh::kWaves, step = 16 * Sh::WT;
+    s->tc = ((w.mrows + step - 1) / step * step + per - 1) / per;
+    s->rot = 0;  // k-blocks in ascending order
+  }
+  // The copies of chunk c and the scales of its token columns.
+  __device__ __attribute__((always_inline)) void issue(unsigned char* stage,
+                                                       const tile::Source<Sh>& s, const Pairs& p,
+                                                       int c) {
+    tile::copies<Sh>(stage, s, woff, wstep, tokens, wave, tile::chunk_byte(c, s.rot, Kdim));
+#pragma unroll
+    for (int t = 0; t < NT; ++t) sx[t] = a.scales[p.scale[t] + (uint32_t)c];
+  }
+  __device__ __attribute__((always_inline)) i32x8 operand(const unsigned char* rows, int tile16,
+                                                          const int (&l)[2]) const {
+    return join(*reinterpret_cast<const u32x4*>(rows + tile16 * 16 * tile::kRowBytes + l[0]),
+                *reinterpret_cast<const u32x4*>(rows + tile16 * 16 * tile::kRowBytes + l[1]));
+  }
+
+  // One chunk, from stage `rds`, with the next chunk's copies into `wrs`
+  // (distinct stages, see dma::step).  sw: the weight scales of the first and
+  // second half of the wave's rows.
+  template <int NTW>
+  __device__ __attribute__((always_inline)) void chunk(unsigned char* __restrict__ wrs,
+                                                       const unsigned char* __restrict__ rds,
+                                                       const tile::Source<Sh>& cs,
+                                                       const Pairs& cp, int cc, float sw0,
+                                                       float sw1, f32x4 (&acc)[NG][NTW]) {
+    float s[NTW];
+#pragma unroll
+    for (int t = 0; t < NTW; ++t) s[t] = sx[t];
+    if (cc >= 0) issue(wrs, cs, cp, cc);
+    const unsigned char* ts = rds + Sh::kRows * tile::kRowBytes;
+    i32x8 tf[NTW], wf = operand(rds, 0, lw);
+#pragma unroll
+    for (int t = 0; t < NTW; ++t) tf[t] = operand(ts, t * Sh::WT, lt);
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+      f32x4 d[NTW];
+#pragma unroll
+      for (int t = 0; t < NTW; ++t) d[t] = mfma_fp8(wf, tf[t]);
+      if (g + 1 < NG) wf = operand(rds, g + 1, lw);
+      const float sw = g < NG / 2 ? sw0 : sw1;
+#pragma unroll
+      for (int t = 0; t < NTW; ++t)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[g][t][e] = acc[g][t][e] + (d[t][e] * s[t]) * sw;
+    }
+  }
+  __device__ __attribute__((always_inline)) void wait() const {
+    dma::wait_vm<0>();
+    dma::lds_barrier();
+  }
+  // At a tile's first chunk, whose copies are older than the stores of the
+  // tile before: those need not be waited for.  Every wave of a tile with n
+  // token tiles a wave makes exactly n * kStores of them.
+  template <int N_ = NT>
+  __device__ __attribute__((always_inline)) void wait_first() const {
+    if constexpr (N_ > 0) {
+      if (stored != N_) return wait_first<N_ - 1>();
+    }
+    dma::wait_vm<N_ * kStores>();
+    dma::lds_barrier();
+  }
+
+  template <int NTW>
+  __device__ __attribute__((always_inline)) void run(tile::Work& w, tile::Source<Sh>& src,
+                                                     Pairs& p, bool* more) {
+    f32x4 acc[NG][NTW];
+#pragma unroll
+    for (int g = 0; g < NG; ++g)
+#pragma unroll
+      for (int t = 0; t < NTW; ++t) acc[g][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const int row0 = panel_row(w) + wr * (kW13 ? NG * 8 : NG * 16);
+    const float* S0 = a.wscale + (size_t)w.slot * a.ws_stride +
+                      (size_t)(row0 / a.block_n) * chunks;
+    const float* S1 = a.wscale + (size_t)w.slot * a.ws_stride +
+                      (size_t)((row0 + (kW13 ? a.I : NG * 8)) / a.block_n) * chunks;
+    tile::Work nw;
+    tile::Source<Sh> ns;
+    Pairs np;
+    float pw[NTW];
+    wait_first();
+    const bool next = take(&nw);
+    if (next) pairs(nw, &np);
+    if constexpr (!kW13) {
+#pragma unroll
+      for (int t = 0; t < NTW; ++t) pw[t] = a.topk_w[p.out[t]];
+    }
+    auto step = [&](const tile::Source<Sh>& cs, const Pairs& cp, int cc, int c)
+                    __attribute__((always_inline)) {
+      chunk<NTW>(smem + (~q & 1) * Sh::kStage, smem + (q & 1) * Sh::kStage, cs, cp, cc, S0[c],
+                 S1[c], acc);
+      ++q;
+    };
+    step(src, p, 1, 0);
+    wait();
+    if (next) source(nw, np, &ns);
+    for (int c = 1; c < chunks - 1; ++c) {
+      step(src, p, c + 1, c);
+      wait();
+    }
+    if (next) place_scales(np);
+    step(ns, np, next ? 0 : -1, chunks - 1);
+    // columns past mrows hold, and store again, the last token's values
+#pragma unroll
+    for (int t = 0; t < NTW; ++t) {
+      if constexpr (kW13) {
+        uint16_t* o = a.out + (size_t)p.out[t] * a.I + row0 + (lane >> 4) * 4;
+#pragma unroll
+        for (int g = 0; g < NG / 2; ++g) {
+          store_act4(o + g * 16, acc[g][t], acc[g + NG / 2][t]);
+          __builtin_amdgcn_sched_barrier(0);  // one store's temporaries at a time
+        }
+      } else {
+        uint16_t* o = a.out + (size_t)p.out[t] * a.H + row0 + (lane >> 4) * 4;
+#pragma unroll
+        for (int g = 0; g < NG; ++g)
+          store_bf16x4(o + g * 16, acc[g][t][0] * pw[t], acc[g][t][1] * pw[t],
+                       acc[g][t][2] * pw[t], acc[g][t][3] * pw[t]);
+      }
+    }
+    stored = NTW;
+    w = nw;
+    src = ns;
+    p = np;
+    *more = next;
+  }
+};
+
+template <typename Sh, bool kW13>
+__global__ __launch_bounds__(64 * Sh::kWaves)
+__attribute__((amdgpu_waves_per_eu(Sh::kWaves / 4, Sh::kWaves / 4))) void fp8_tile_kernel(
+    Fp8TileArgs a) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  tile::Table* tab = reinterpret_cast<tile::Table*>(smem + Sh::kTable);
+  Fp8TileLoop<Sh, kW13> L{a, smem, tab};
+  L.N = kW13 ? 2 * a.I : a.H;
+  L.Kdim = kW13 ? a.H : a.I;
+  L.npanels = L.N / Sh::kRows;
+  L.chunks = L.Kdim / kKB;
+  L.wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  L.lane = threadIdx.x & 63;
+  L.wr = L.wave % Sh::WR;
+  L.wt = L.wave / Sh::WR;
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const int cb = 2 * (L.lane >> 4) + u;
+    L.lw[u] = dma::swz(L.wr * Sh::NG * 16 + (L.lane & 15), cb);
+    L.lt[u] = dma::swz(L.wt * 16 + (L.lane & 15), cb);
+  }
+  L.tokens = {a.A, (uint32_t)a.rows * (uint32_t)L.Kdim};
+  static_assert(Sh::kWaves * tile::kRowsPerCopy == 64 && Sh::NG % 4 == 0, "weight_row(64 i + r) is weight_row(64 i) + weight_row(r) for r < 64");
+  L.woff = (uint32_t)L.weight_row(L.copy_row(0)) * (uint32_t)L.Kdim +
+           (((L.lane % dma::kLanesPerRow) ^ (L.copy_row(0) & 7)) << 4);
+#pragma unroll
+  for (int i = 0; i < Sh::kWCopies; ++i)
+    L.wstep[i] = (uint32_t)L.weight_row(i * Sh::kWaves * tile::kRowsPerCopy) * (uint32_t)L.Kdim;
+  if (L.wave == 0) tile::fill_table(tab, a.counts, a.nslots, Sh::kToks);
+  __syncthreads();
+  tile::Work w;
+  bool more = L.take(&w);
+  if (!more) return;
+  tile::Source<Sh> src;
+  typename Fp8TileLoop<Sh, kW13>::Pairs p;
+  L.pairs(w, &p);
+  L.source(w, p, &src);
+  L.place_scales(p);
+  L.issue(smem, src, p, 0);
+  while (more) {
+    const int nt = (w.mrows + 16 * Sh::WT - 1) / (16 * Sh::WT);
+    if (nt == 1)
+      L.template run<1>(w, src, p, &more);
+    else if (nt == 2)
+      L.template run<2>(w, src, p, &more);
+    else if (nt == 3)
+      L.template run<3>(w, src, p, &more);
+    else if (Sh::NT == 4 || nt == 4)
+      L.template run<4>(w, src, p, &more);
+    else if (nt == 5)
+      L.template run<(Sh::NT > 4 ? 5 : 4)>(w, src, p, &more);
+    else
+      L.template run<(Sh::NT > 4 ? 6 : 4)>(w, src, p, &more);
+  }
+}
+
+template <typename Sh, bool kW13>
+hipError_t launch_fp8_tile(const Fp8TileArgs& a, hipStream_t st, hipEvent_t e0, hipEvent_t e1) {
+  constexpr unsigned lds = Sh::kTable + sizeof(tile::Table);
+  static_assert(lds <= kMaxLds, "LDS per block");
+  static std::atomic<uint64_t> big{0};
+  hipError_t e = allow_lds(&fp8_tile_kernel<Sh, kW13>, lds, lds, &big);
+  if (e != hipSuccess) return e;
+  launch_timed_lds(fp8_tile_kernel<Sh, kW13>, dim3(tile::kBlocks), dim3(64 * Sh::kWaves), lds, st,
+                   e0, e1, a);
+  return hipSuccess;
+}
+
 // out[t, h] = moe_sum over k ascending of y[(t, k), h]: bf16 adds for K in
-// {2, 3, 4}, else one float32 sum rounded once.  grid = (ceil(H / 256), T).
+// {2, 3, 4}, else one float32 sum rounded once.  grid = (ceil(H / 2048), T),
+// 8 columns a thread, the loads of up to kCombineK pairs issued before their
+// sums (the kernel streams P * H bf16 values; one column a thread and one
+// load at a time held it at 2.3 TB/s, 59 us at 4096 tokens of the Qwen3
+// shape).
+constexpr int kCombineK = 8;
+
 __global__ __launch_bounds__(256) void fp8_combine_kernel(const uint16_t* __restrict__ y, int H,
                                                           int K, int nslots,
                                                           const int32_t* __restrict__ slots,
                                                           uint16_t* __restrict__ out) {
   const int t = blockIdx.y;
-  const int h = blockIdx.x * 256 + threadIdx.x;
+  const int h = (blockIdx.x * 256 + threadIdx.x) * 8;
   if (h >= H) return;
   const bool bf16_adds = K >= 2 && K <= 4;
-  float sum = 0.f;
-  for (int k = 0; k < K; ++k) {
-    const int p = t * K + k;
-    const int s = slots[p];
-    const float v = (s < 0 || s >= nslots) ? 0.f : bf16f(y[(size_t)p * H + h]);
-    sum = bf16_adds ? round_bf16(sum + v) : sum + v;
+  float sum[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) sum[j] = 0.f;
+  for (int k0 = 0; k0 < K; k0 += kCombineK) {
+    u32x4 v[kCombineK];
+    bool ok[kCombineK];
+#pragma unroll
+    for (int k = 0; k < kCombineK; ++k) {
+      if (k0 + k < K) {
+        const int p = t * K + k0 + k;
+        const int s = slots[p];
+        ok[k] = s >= 0 && s < nslots;
+        v[k] = *reinterpret_cast<const u32x4*>(y + (size_t)p * H + h);
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < kCombineK; ++k) {
+      if (k0 + k < K) {
+        float f[8];
+        unpack_bf16x8(v[k], f);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          const float a = sum[j] + (ok[k] ? f[j] : 0.f);
+          sum[j] = bf16_adds ? round_bf16(a) : a;
+        }
+      }
+    }
   }
-  out[(size_t)t * H + h] = bf16_rne(sum);
+  uint16_t* o = out + (size_t)t * H + h;
+  if ((uintptr_t)out % 16 == 0) {  // H is a multiple of 128
+    u32x4 r;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      r[j] = (uint32_t)bf16_rne(sum[2 * j]) | ((uint32_t)bf16_rne(sum[2 * j + 1]) << 16);
+    *reinterpret_cast<u32x4*>(o) = r;
+  } else {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) o[j] = bf16_rne(sum[j]);
+  }
 }
 
 // Work buffer of the grouped path (bytes, each piece 256-byte aligned).
@@ -1736,6 +2070,21 @@ const char* fp8_unsupported(int H, int I, int K, int block_n, int block_k) {
   return nullptr;
 }
 
+// Calls of at least this many pairs per slot take the block tiles, as the
+// bf16 path does and for its reason.  Measured at the Qwen3-FP8 shape, 64-token
+// blocks against tiles, w13 + w2 (us): 48 / 56 / 64 / 128 / 512 pairs per slot
+// 160 / 171 / 210 / 349 / 1197 against 179 / 176 / 189 / 232 / 706.
+constexpr int kFp8TileMinPairs = 60;
+
+// Whether a call takes the block tiles: 256-row panels of H, a wave's 64 rows
+// within one scale block, k loops of two chunks or more, 32-bit row offsets.
+bool fp8_tile_call(int P, int T, int H, int I, int nslots, int block_n, uintptr_t addresses) {
+  const uint64_t lim = 1ull << 32;
+  return addresses % 16 == 0 && (int64_t)P >= (int64_t)kFp8TileMinPairs * nslots &&
+         nslots <= kMaxExperts && H % 256 == 0 && I >= 2 * kKB && block_n % 64 == 0 &&
+         (uint64_t)T * H < lim && (uint64_t)P * I < lim && (uint64_t)I * H * 2 < lim;
+}
+
 // The LDS-staged kernels with the activation quantisation between them.
 template <int S13, int S2, int NP2>
 bool launch_grouped_dma(const uint8_t* xq, const float* xs, uint8_t* aq, float* as, int T, int H,
@@ -1839,10 +2188,29 @@ int experts_fp8_grouped(const void* x, int T, int H, int I, int K, const float* 
   auto dma = np2 == kNP ? &launch_grouped_dma<2, 3, kNP>
              : np2 == 2 ? &launch_grouped_dma<2, 3, 2>
                         : &launch_grouped_dma<2, 3, 1>;
+  if (fp8_tile_call(P, T, H, I, nslots, block_n,
+                    (uintptr_t)w13 | (uintptr_t)w2 | w13_stride | w2_stride)) {
+    using Sh = tile::Shape<2, 4, 8, 4>;
+    const Fp8TileArgs t13{xq,  xs,         H,   I,         K,       P,  T, nslots, lists, counts,
+                          topk_w, a13, w13_stride, s13, s13_stride, block_n, ab};
+    const Fp8TileArgs t2{aq,  as,        H,  I,         K,       P, P, nslots, lists, counts,
+                         topk_w, a2, w2_stride, s2, s2_stride, block_n, y};
+    WISP_HIP_TRY((launch_fp8_tile<Sh, true>(t13, st, ev ? ev->ev[0] : nullptr,
+                                            ev ? ev->ev[1] : nullptr)));
+    const long jobs2 = (long)P * (I / kKB);
+    hipLaunchKernelGGL(quant_groups_kernel<uint16_t>, dim3((unsigned)((jobs2 + 15) / 16)),
+                       dim3(256), 0, st, (const uint16_t*)act, P, I, aq, as);
+    WISP_HIP_TRY((launch_fp8_tile<Sh, false>(t2, st, ev ? ev->ev[2] : nullptr,
+                                             ev ? ev->ev[3] : nullptr)));
+    hipLaunchKernelGGL(fp8_combine_kernel, dim3((H + 2047) / 2048, T), dim3(256), 0, st, y, H, K,
+                       nslots, slots, (uint16_t*)out);
+    WISP_HIP_TRY(hipGetLastError());
+    return WISP_OK;
+  }
   if (T > 16 && dma(xq, xs, aq, as, T, H, I, K, nslots, lists, counts, topk_w,
                     (const uint8_t*)w13, w13_stride, s13, s13_stride, (const uint8_t*)w2,
                     w2_stride, s2, s2_stride, block_n, (uint16_t*)act, y, st, ev)) {
-    hipLaunchKernelGGL(fp8_combine_kernel, dim3((H + 255) / 256, T), dim3(256), 0, st, y, H, K,
+    hipLaunchKernelGGL(fp8_combine_kernel, dim3((H + 2047) / 2048, T), dim3(256), 0, st, y, H, K,
                        nslots, slots, (uint16_t*)out);
     WISP_HIP_TRY(hipGetLastError());
     return WISP_OK;
@@ -1865,7 +2233,7 @@ int experts_fp8_grouped(const void* x, int T, int H, int I, int K, const float* 
     else WISP_GROUPED(4, 1);
   }
 #undef WISP_GROUPED
-  hipLaunchKernelGGL(fp8_combine_kernel, dim3((H + 255) / 256, T), dim3(256), 0, st, y, H, K,
+  hipLaunchKernelGGL(fp8_combine_kernel, dim3((H + 2047) / 2048, T), dim3(256), 0, st, y, H, K,
                      nslots, slots, (uint16_t*)out);
   WISP_HIP_TRY(hipGetLastError());
   return WISP_OK;

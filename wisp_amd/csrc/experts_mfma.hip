@@ -373,7 +373,7 @@ struct TileLoop {
   const tile::Table* tab;
   int N, Kdim, npanels, chunks;
   int wave, lane, wr, wt;
-  uint32_t woff[Sh::kWCopies];
+  uint32_t woff, wstep[Sh::kWCopies];
   // this lane's place, in a stage's weight (token) rows, of the fragment of
   // its wave's first row group (token tile) for either k-step
   int lw[2], lt[2];
@@ -433,7 +433,7 @@ struct TileLoop {
   }
   __device__ __attribute__((always_inline)) void issue(unsigned char* stage,
                                                        const tile::Source<Sh>& s, int c) const {
-    tile::copies<Sh>(stage, s, woff, tokens, wave, tile::chunk_byte(c, s.rot, Kdim * 2));
+    tile::copies<Sh>(stage, s, woff, wstep, tokens, wave, tile::chunk_byte(c, s.rot, Kdim * 2));
   }
   template <int NT>
   __device__ __attribute__((always_inline)) void read_t(const unsigned char* stage, int u, int i,
@@ -594,12 +594,12 @@ __attribute__((amdgpu_waves_per_eu(Sh::kWaves / 4, Sh::kWaves / 4))) void mfma_t
     L.lt[u] = dma::swz(L.wt * 16 + (L.lane & 15), u * 4 + (L.lane >> 4));
   }
   L.tokens = {a.A, (uint32_t)(kW13 ? a.P / a.K : a.P) * (uint32_t)(L.Kdim * 2)};
+  static_assert(Sh::kWaves * tile::kRowsPerCopy == 64 && Sh::NG % 4 == 0, "weight_row(64 i + r) is weight_row(64 i) + weight_row(r) for r < 64");
+  L.woff = (uint32_t)L.weight_row(L.copy_row(0)) * (uint32_t)(L.Kdim * 2) +
+           (((L.lane % dma::kLanesPerRow) ^ (L.copy_row(0) & 7)) << 4);
 #pragma unroll
-  for (int i = 0; i < Sh::kWCopies; ++i) {
-    const int r = L.copy_row(i);
-    L.woff[i] = (uint32_t)L.weight_row(r) * (uint32_t)(L.Kdim * 2) +
-                (((L.lane % dma::kLanesPerRow) ^ (r & 7)) << 4);
-  }
+  for (int i = 0; i < Sh::kWCopies; ++i)
+    L.wstep[i] = (uint32_t)L.weight_row(i * Sh::kWaves * tile::kRowsPerCopy) * (uint32_t)(L.Kdim * 2);
   if (L.wave == 0) tile::fill_table(tab, a.counts, a.nslots, Sh::kToks);
   __syncthreads();
   tile::Work w;
@@ -738,8 +738,6 @@ hipError_t launch_dma(const uint16_t* x, int H, int I, int K, int P, int nslots,
                                                       w2_stride, y, st, e2, e3);
 }
 
-constexpr int kTileBlocks = 256;  // persistent blocks: one per CU
-
 template <typename Sh, bool kW13>
 hipError_t launch_tile(const TileArgs& a, hipStream_t st, hipEvent_t e0, hipEvent_t e1) {
   constexpr unsigned lds = Sh::kTable + sizeof(tile::Table);
@@ -747,7 +745,7 @@ hipError_t launch_tile(const TileArgs& a, hipStream_t st, hipEvent_t e0, hipEven
   static std::atomic<uint64_t> big{0};
   hipError_t e = allow_lds(&mfma_tile_kernel<Sh, kW13>, lds, lds, &big);
   if (e != hipSuccess) return e;
-  launch_timed_lds(mfma_tile_kernel<Sh, kW13>, dim3(kTileBlocks), dim3(64 * Sh::kWaves), lds, st,
+  launch_timed_lds(mfma_tile_kernel<Sh, kW13>, dim3(tile::kBlocks), dim3(64 * Sh::kWaves), lds, st,
                    e0, e1, a);
   return hipSuccess;
 }
@@ -764,7 +762,7 @@ hipError_t launch_tiles(const TileArgs& a, hipStream_t st, hipEvent_t e0, hipEve
   const int busy = std::min(a.P, a.nslots);
   const int64_t works = (int64_t)((kW13 ? 2 * a.I : a.H) / Big::kRows) * busy *
                         ((a.P / busy + Big::kToks - 1) / Big::kToks);
-  return works >= kTileBlocks ? launch_tile<Big, kW13>(a, st, e0, e1)
+  return works >= tile::kBlocks ? launch_tile<Big, kW13>(a, st, e0, e1)
                               : launch_tile<Small, kW13>(a, st, e0, e1);
 }
 

@@ -41,10 +41,11 @@ struct Work {
   int slot, panel, m0, mrows;
 };
 
-// Blocks are persistent: block b takes works work_of(b, 0), work_of(b, 1),
+// Blocks are persistent, one per CU: block b takes works work_of(b, 0), work_of(b, 1),
 // ...  Blocks go to the XCDs round-robin, and each XCD takes runs of kRun
 // consecutive works, so blocks that read the same weights or tokens share
 // an L2.
+constexpr int kBlocks = 256;
 constexpr int kRun = 32;
 __device__ inline int work_of(int b, int j) {
   const int i = (b >> 3) + j * ((int)gridDim.x >> 3);
@@ -114,8 +115,18 @@ struct Range {
   uint32_t bytes;
 };
 
-// 16 (4) bytes per lane from r, lane offset voff plus the wave's offset o,
-// into LDS at dst + 16 (4) * lane.
+// r in scalar registers (it is the same for the whole wave, which the
+// compiler does not always see).
+__device__ __attribute__((always_inline)) inline Range scalar(const Range& r) {
+  const uint64_t p = (uint64_t)r.p;
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)p);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(p >> 32));
+  return Range{(const void*)(((uint64_t)hi << 32) | lo),
+               (uint32_t)__builtin_amdgcn_readfirstlane((int)r.bytes)};
+}
+
+// 16 bytes per lane from r, lane offset voff plus the wave's offset o, into
+// LDS at dst + 16 * lane.
 #ifdef __HIP_DEVICE_COMPILE__  // the host pass does not know these builtins
 #define WISP_COPY_TO_LDS(size)                                                                   \
   __builtin_amdgcn_raw_ptr_buffer_load_lds(                                                      \
@@ -149,16 +160,17 @@ __device__ inline int chunk_byte(int c, int rot, int row_bytes) {
 
 template <typename Sh>
 __device__ __attribute__((always_inline)) inline void copies(
-    unsigned char* st, const Source<Sh>& src, const uint32_t (&woff)[Sh::kWCopies],
-    const Range& tokens, int wave, int o) {
+    unsigned char* st, const Source<Sh>& src, uint32_t woff,
+    const uint32_t (&wstep)[Sh::kWCopies], const Range& tokens, int wave, int o) {
+  const Range wr = scalar(src.w), tr = scalar(tokens);
+  o = __builtin_amdgcn_readfirstlane(o);
 #pragma unroll
   for (int i = 0; i < Sh::kWCopies; ++i)
-    copy16(src.w, woff[i], o, st + (i * Sh::kWaves + wave) * 1024);
+    copy16(wr, woff, o + (int)wstep[i], st + (i * Sh::kWaves + wave) * 1024);
 #pragma unroll
   for (int i = 0; i < Sh::kTCopies; ++i)
     if (i < src.tc)
-      copy16(tokens, src.toff[i], o,
-               st + Sh::kRows * kRowBytes + (i * Sh::kWaves + wave) * 1024);
+      copy16(tr, src.toff[i], o, st + Sh::kRows * kRowBytes + (i * Sh::kWaves + wave) * 1024);
 }
 
 }  // namespace tile
