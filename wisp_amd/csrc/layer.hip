@@ -658,6 +658,26 @@ int experts(Layer& L, const void* x, int T, int K, const float* w, const int32_t
   return w2(L, act, T, K, w, slots, out, st, nullptr, nullptr);
 }
 
+// Whether a call that auto_algo gives the decode kernels is faster on the
+// grouped ones because its tokens share experts.  Uniform routing over E
+// experts makes T tokens meet D = E (1 - (1 - K / E)^T) distinct ones; the
+// decode kernels stream T * K experts' weights, the grouped ones D and three
+// small launches more.  Measured, T * K / D and decode against grouped (us):
+// bf16 Mixtral (8 experts, top-2) 1.14 / 1.30 / 1.46 / 1.82 / 2.22 at 2 / 3 /
+// 4 / 6 / 8 tokens, 211 / 312 / 409 / 613 / 821 against 230 / 292 / 309 /
+// 363 / 405; bf16 Qwen3 (128, top-8) 1.39 / 1.47 at 12 / 14 tokens, 133 / 153
+// against 140 / 144.  Block-FP8 Qwen3, 1.24 / 1.39 / 1.55 at 8 / 12 / 16
+// tokens: 90 / 107 / 125 against 94 / 96 / 109.  Like auto_algo it depends on
+// the shape and the token count alone.
+bool shares_experts(int dtype, int H, int I, int E, int T, int K) {
+  if (dtype == WISP_F32 || T < 2 || K > E) return false;
+  if (dtype == WISP_BF16 && !mfma_supported(H, I)) return false;
+  double absent = 1.0;
+  for (int t = 0; t < T && absent > 1e-6; ++t) absent *= 1.0 - (double)K / E;
+  const double ratio = dtype == WISP_BF16 ? 1.45 : 1.3;
+  return (double)T * K >= ratio * E * (1.0 - absent);
+}
+
 // The expert algorithm of a layer call (-1: the request does not cover it).
 // Decided before the pager runs, so a call the kernels cannot compute fails
 // without touching the pager state.
@@ -1021,7 +1041,13 @@ extern "C" int wisp_layer_forward(void* handle, const void* x, const void* logit
       return WISP_ERR_UNSUPPORTED;
     }
   }
-  const int a = choose_algo(*L, algo, T, K);
+  int a = choose_algo(*L, algo, T, K);
+  // (only with a work buffer for it: callers that size theirs by auto_algo's
+  // choice keep the decode kernels)
+  if (algo == WISP_ALGO_AUTO && a == WISP_ALGO_GEMV &&
+      shares_experts(d.dtype, d.hidden, d.inter, d.num_experts, T, K) &&
+      work_ok(*L, WISP_ALGO_MFMA, T, K, ws))
+    a = WISP_ALGO_MFMA;
   if (a < 0) {
     wisp_set_last_error("no expert kernel covers this call (shape, top_k or requested "
                         "algorithm)", "wisp_layer_forward");
