@@ -7,6 +7,7 @@ import torch
 from oracle.moe import moe_forward, route
 from oracle.pager import PagerOracle
 from tests._util import fixture_matches, load_golden, oracle_trace_matches
+from wisp_amd import _lib
 from wisp_amd import workloads as W
 from wisp.integrations.vllm.fused_moe import WispMoEState
 from wisp_amd.record import parse_record
@@ -664,3 +665,50 @@ def test_bfloat16_router_logits(monkeypatch, fused):
             assert np.allclose(w_gpu.cpu().numpy(), w_ref, rtol=2e-6, atol=1e-7), (key, t, T)
             assert st.last_slots.cpu().tolist() == ora_res["slots"], (key, t, T)
             assert st.slot_to_expert == ora.slot_to_expert and st.lru_tick == ora.lru_tick
+
+
+# rows of 1, 2, 4 and 8 chunks a lane; one expert, fewer and more than 64, all
+# 128; I with a partial block of rows; the largest fused call and one more
+@pytest.mark.parametrize("dtype,H,I,E,K,tokens", [
+    (torch.float32, 256, 64, 1, 1, (1, 8)), (torch.float32, 512, 256, 16, 2, (1, 4, 8, 9)),
+    (torch.bfloat16, 512, 88, 65, 5, (1, 3, 8, 9)), (torch.bfloat16, 1024, 256, 60, 4, (2, 5)),
+    (torch.bfloat16, 2048, 128, 128, 8, (1, 7, 8)), (torch.bfloat16, 4096, 64, 12, 3, (1, 2)),
+])
+@pytest.mark.parametrize("logits_dtype", [torch.float32, torch.bfloat16])
+def test_resident_calls_routed_in_the_w13_launch(dtype, H, I, E, K, tokens, logits_dtype):
+    """Small resident calls: weights and ids equal the router kernel's bit for
+    bit (also among tied logits), the output the decode kernels' on those
+    ids, and the call counter ticks once a call."""
+    g = torch.Generator().manual_seed(H + E)
+    w13 = (torch.randn((E, 2 * I, H), generator=g) * 0.05).to(dtype).pin_memory()
+    w2 = (torch.randn((E, H, I), generator=g) * 0.05).to(dtype).pin_memory()
+    st = WispMoEState(w13, w2, E, "resident", DEV, 0)
+    st.prime_identity()
+    calls = 0
+    for T in tokens:
+        x = torch.randn((T, H), generator=g).to(dtype).to(DEV)
+        for lg in (torch.randn((T, E), generator=g),
+                   torch.randint(-2, 3, (T, E), generator=g).float()):
+            for renorm in (True, False):
+                lgd = lg.to(logits_dtype).to(DEV)
+                out = st.forward(x, lgd, K, renorm, algo=_lib.WISP_ALGO_GEMV)
+                calls += 1
+                w, ids = st.last_topk
+                wr = torch.empty_like(w)
+                ir = torch.empty_like(ids)
+                code = _lib.WISP_F32 if logits_dtype == torch.float32 else _lib.WISP_BF16
+                _lib.check(_lib.lib().wisp_route_topk_softmax(
+                    lgd.data_ptr(), code, T, E, K, int(renorm), wr.data_ptr(), ir.data_ptr(),
+                    None, _lib.stream_handle()), "route")
+                act = torch.empty(T * K * I, dtype=dtype, device=DEV)
+                ref = torch.empty_like(out)
+                _lib.check(_lib.lib().wisp_moe_experts(
+                    x.data_ptr(), _lib.WISP_F32 if dtype == torch.float32 else _lib.WISP_BF16, T,
+                    H, I, K, wr.data_ptr(), ir.data_ptr(), E, st.scratch_w13.data_ptr(),
+                    st.scratch_w13.stride(0), st.scratch_w2.data_ptr(), st.scratch_w2.stride(0),
+                    act.data_ptr(), ref.data_ptr(), None, 0, _lib.WISP_ALGO_GEMV,
+                    _lib.stream_handle()), "experts")
+                torch.cuda.synchronize()
+                assert torch.equal(ids, ir) and torch.equal(w, wr), (T, renorm)
+                assert torch.equal(bits(out), bits(ref)), (T, renorm)
+    assert st.stats_forward == calls

@@ -187,6 +187,66 @@ __global__ __launch_bounds__(256) void w13_silu_kernel(const T* __restrict__ x, 
 }
 
 // ---------------------------------------------------------------------------
+// Kernel A for a resident layer's smallest calls, with the router in front:
+// block (i, pair) routes its own token (wave 0, and only as many rounds as
+// its pair's place in the top-k needs) while all four waves load their part
+// of x, then runs the pair's rows.  The block of row 0 of a token's last pair
+// has all of its choices and writes them for w2.  E <= 128, whole rows.
+// Such a call is bound by its launches: the router's took 3.8 us for one
+// wave's work.  Measured, separate launches against this one (us per call):
+// Qwen3 18.9 -> 16.5 / 30.2 -> 28.7 / 50.8 -> 49.5 / 81.5 -> 80.2 at 1 / 2 /
+// 4 / 7 tokens, the fp32 toy layer 17.1 -> 14.5; with eight chunks a lane
+// (Mixtral) 110.7 -> 110.0 at one token but 210.2 -> 210.9 at two, so there
+// only one-token calls take it.
+// ---------------------------------------------------------------------------
+constexpr int kRouteW13Tokens = 8;
+
+template <typename TL>
+struct RouteArgs {
+  const TL* logits;  // [T][E]
+  int E, renorm;
+  float* w;          // [T][K]
+  int32_t* ids;
+  int64_t* forward;  // layer-call counter
+};
+
+template <typename T, typename TL, int CH>
+__global__ __launch_bounds__(256) void route_w13_kernel(const T* __restrict__ x, int H, int I,
+                                                        int K, RouteArgs<TL> r,
+                                                        const T* __restrict__ w13,
+                                                        size_t w13_stride, T* __restrict__ act) {
+  __shared__ RoutePos pos;
+  __shared__ int32_t chosen;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int pair = blockIdx.y, t = pair / K, k = pair - t * K;
+  float raw[2];
+  if (wave == 0) route_load_logits<TL, 2>(r.logits + (size_t)t * r.E, r.E, lane, raw);
+  uint4 xv[CH], wg[CH], wu[CH];
+  load_row<T, CH, true, false>(x + (size_t)t * H, 0, lane, xv);
+  if (wave == 0) {
+    const bool writes = blockIdx.x == 0 && k == K - 1;
+    float w;
+    int id;
+    route_token_loaded<2>(raw, r.E, k + 1, r.renorm, lane, true, &w, &id, pos, nullptr, writes);
+    if (lane == k) chosen = id;
+    if (writes && lane < K) {
+      r.w[(size_t)t * K + lane] = w;
+      r.ids[(size_t)t * K + lane] = id;
+    }
+    if (writes && t == 0 && lane == 0) r.forward[0] += 1;
+  }
+  block_lds_sync();
+  const int s = __builtin_amdgcn_readfirstlane(chosen);
+  const int i = blockIdx.x * 4 + wave;
+  if (i >= I) return;
+  const T* W = w13 + (size_t)s * w13_stride;
+  load_row<T, CH, true, true>(W + (size_t)i * H, 0, lane, wg);
+  load_row<T, CH, true, true>(W + (size_t)(I + i) * H, 0, lane, wu);
+  const float v = swiglu_rows<T, CH, uint4>(wg, wu, xv);
+  if (lane == 0) store_elem(act + (size_t)pair * I + i, v);
+}
+
+// ---------------------------------------------------------------------------
 // Kernel A': page-in and w13 in one launch, for one-token calls on the
 // copy-kernel engine (a token's routed experts are distinct, so each expert
 // serves exactly one pair).
@@ -822,6 +882,27 @@ int dispatch_pagein_w13(const PageInArgs& a, const FusedW13Args& f, hipStream_t 
   return WISP_OK;
 }
 
+template <typename T, typename TL>
+int dispatch_route_w13(const T* x, int T_, int H, int I, int K, const RouteArgs<TL>& r,
+                       const T* w13, size_t w13_stride, T* act, hipStream_t st, hipEvent_t e0,
+                       hipEvent_t e1) {
+  const dim3 grid((I + 3) / 4, T_ * K);
+#define WISP_ROUTE_W13(CH)                                                              \
+  case CH:                                                                              \
+    launch_timed(route_w13_kernel<T, TL, CH>, grid, dim3(256), st, e0, e1, x, H, I, K, r, \
+                 w13, w13_stride, act);                                                 \
+    break
+  switch (w13_chunks<T>(H)) {
+    WISP_ROUTE_W13(1);
+    WISP_ROUTE_W13(2);
+    WISP_ROUTE_W13(4);
+    WISP_ROUTE_W13(8);
+    default: return WISP_ERR_UNSUPPORTED;
+  }
+#undef WISP_ROUTE_W13
+  return WISP_OK;
+}
+
 // Kernel A'' for whole rows of 2 or 4 chunks per lane (the other shapes keep
 // the separate pager launch: at 8 chunks the launch's 80 VGPRs spill).
 template <typename T, typename TL>
@@ -945,6 +1026,42 @@ int decode_w13(const PageInArgs& a, const void* x, int dtype, int logits_dtype, 
   if (rc != WISP_OK) {
     wisp_set_last_error("hidden size outside the fused decode launch's coverage",
                         "decode w13 kernel");
+    return rc;
+  }
+  WISP_HIP_TRY(hipGetLastError());
+  return WISP_OK;
+}
+
+// Whether route_w13 serves a resident layer's call (the router instance of
+// two logits a lane, whole rows of 1, 2, 4 or 8 chunks).
+bool route_w13_supported(int dtype, int T_, int H, int E, int K) {
+  const int V = dtype == WISP_F32 ? 4 : 8;
+  const int ch = H / V / 64;
+  return T_ >= 1 && T_ <= (ch == 8 ? 1 : kRouteW13Tokens) && E <= 128 && K <= E &&
+         H % (64 * V) == 0 && (ch == 1 || ch == 2 || ch == 4 || ch == 8) &&
+         gemv_supported(dtype, H, K);
+}
+
+int route_w13(const void* logits, int logits_dtype, int E, int renorm, float* topk_w,
+              int32_t* topk_ids, int64_t* forward, const void* x, int dtype, int T_, int H, int I,
+              int K, const void* w13, size_t w13_stride, void* act, hipStream_t st, hipEvent_t e0,
+              hipEvent_t e1) {
+  int rc;
+  const RouteArgs<float> rf{(const float*)logits, E, renorm, topk_w, topk_ids, forward};
+  const RouteArgs<uint16_t> rb{(const uint16_t*)logits, E, renorm, topk_w, topk_ids, forward};
+  const bool lf = logits_dtype == WISP_F32;
+  if (dtype == WISP_F32)
+    rc = lf ? dispatch_route_w13((const float*)x, T_, H, I, K, rf, (const float*)w13, w13_stride,
+                                 (float*)act, st, e0, e1)
+            : dispatch_route_w13((const float*)x, T_, H, I, K, rb, (const float*)w13, w13_stride,
+                                 (float*)act, st, e0, e1);
+  else
+    rc = lf ? dispatch_route_w13((const uint16_t*)x, T_, H, I, K, rf, (const uint16_t*)w13,
+                                 w13_stride, (uint16_t*)act, st, e0, e1)
+            : dispatch_route_w13((const uint16_t*)x, T_, H, I, K, rb, (const uint16_t*)w13,
+                                 w13_stride, (uint16_t*)act, st, e0, e1);
+  if (rc != WISP_OK) {
+    wisp_set_last_error("hidden size outside the fused router's coverage", "route + w13 kernel");
     return rc;
   }
   WISP_HIP_TRY(hipGetLastError());

@@ -42,7 +42,8 @@
 // side streams only pay off when there is independent work to overlap.
 //
 // Resident mode (cap == E, identity map) skips the pager and the sync and
-// reads expert e from slot e.
+// reads expert e from slot e; its calls of a few tokens route in the w13
+// launch: [route + w13] [w2].
 #include <string.h>
 
 #include <string>
@@ -72,6 +73,11 @@ int launch_pager(const int32_t* ids, const void* logits, int logits_dtype, int r
 int gemv_w13(const void* x, int dtype, int T, int H, int I, int K, const int32_t* slots,
              int nslots, const void* w13, size_t w13_stride, void* act, hipStream_t st,
              hipEvent_t ev_start, hipEvent_t ev_stop, const int32_t* pair_filter, int want);
+bool route_w13_supported(int dtype, int T, int H, int E, int K);
+int route_w13(const void* logits, int logits_dtype, int E, int renorm, float* topk_w,
+              int32_t* topk_ids, int64_t* forward, const void* x, int dtype, int T, int H, int I,
+              int K, const void* w13, size_t w13_stride, void* act, hipStream_t st, hipEvent_t e0,
+              hipEvent_t e1);
 int pagein_w13(const PageInArgs& a, const void* x, int dtype, int T, int H, int I, int K,
                const int32_t* flags, const void* w13, size_t w13_stride, void* act,
                hipStream_t st, hipEvent_t ev_start, hipEvent_t ev_stop);
@@ -1062,6 +1068,20 @@ extern "C" int wisp_layer_forward(void* handle, const void* x, const void* logit
 
   L->rec_on_device = false;
   if (d.mode == WISP_MODE_RESIDENT) {
+    if (a == WISP_ALGO_GEMV && !L->fp8 && logits &&
+        (logits_dtype == WISP_F32 || logits_dtype == WISP_BF16) && ws->topk_w && ws->topk_ids &&
+        route_w13_supported(d.dtype, T, d.hidden, d.num_experts, K)) {
+      // [route + w13] [w2]
+      ProfLaunch* p = prof_begin(*L, 0);
+      if (p) L->prof_w13_calls += 1;
+      rc = route_w13(logits, logits_dtype, d.num_experts, renormalize, ws->topk_w, ws->topk_ids,
+                     d.counters + kForward, x, d.dtype, T, d.hidden, d.inter, K, d.scratch_w13,
+                     d.scratch_w13_stride, ws->act, st, p ? p->start : nullptr,
+                     p ? p->stop : nullptr);
+      if (p && rc == WISP_OK) p->pending = true;
+      if (rc != WISP_OK) return rc;
+      return w2(*L, ws->act, T, K, ws->topk_w, ws->topk_ids, out, st, nullptr, nullptr);
+    }
     rc = wisp_route_topk_softmax(logits, logits_dtype, T, d.num_experts, K, renormalize,
                                  ws->topk_w, ws->topk_ids, d.counters + kForward, stream);
     if (rc != WISP_OK) return rc;

@@ -104,11 +104,13 @@ __device__ inline void route_load_logits(const TL* __restrict__ logits_row, int 
 // return (weight, id) of routing position `lane`; other lanes return
 // (0, -1).  `picked` (optional): bit j is set in lane l when expert 64 j + l
 // was chosen.  `pos`: this wave's LDS.  All lanes of the wave must call it,
-// with K <= E (every round then chooses an eligible entry).
+// with K <= E (every round then chooses an eligible entry).  Without
+// `weights` the ids alone are wanted, and weights stay 0.
 template <int VALS>
 __device__ inline void route_token_loaded(const float (&raw)[VALS], int E, int K, int renorm,
                                           int lane, bool active, float* w_out, int* id_out,
-                                          RoutePos& pos, uint32_t* picked = nullptr) {
+                                          RoutePos& pos, uint32_t* picked = nullptr,
+                                          bool weights = true) {
   (void)RouteVals<VALS>();
   const int per = min((E + 63) >> 6, VALS);
   float v[VALS];
@@ -165,6 +167,11 @@ __device__ inline void route_token_loaded(const float (&raw)[VALS], int E, int K
   wave_lds_sync();
   const float m = unrank_bits(first);
   const int my_id = lane < K ? pos.id[lane] : -1;
+  if (picked) *picked = sel;
+  if (!weights) {
+    *id_out = my_id;
+    return;
+  }
   const float my_v = lane < K ? pos.v[lane] : 0.f;
   float ls = 0.f;
 #pragma unroll
@@ -177,7 +184,6 @@ __device__ inline void route_token_loaded(const float (&raw)[VALS], int E, int K
     *w_out = p;
     *id_out = my_id;
   }
-  if (picked) *picked = sel;
 }
 
 template <typename TL, int VALS>
