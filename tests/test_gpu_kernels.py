@@ -289,6 +289,25 @@ def test_experts_gemv_bf16(T, H, I, E, K):
     assert rel_err(out, moe_forward(x, w, ids, w13, w2, act_round="bf16")) < 4e-3
 
 
+# Calls of two or more tokens and at most 128 pairs read an expert's w13 rows
+# once for all of its pairs: pair counts around the 64 lanes of a wave and at
+# the limit and one over it, one expert for all, a pair without a slot.
+@pytest.mark.parametrize("T,K,E", [(2, 1, 1), (8, 8, 16), (13, 5, 9), (16, 8, 24), (43, 3, 7),
+                                    (64, 2, 2)])
+@pytest.mark.parametrize("dtype,H,I", [(torch.bfloat16, 2048, 70), (torch.float32, 320, 33)])
+def test_gemv_bytes_with_shared_experts(T, K, E, dtype, H, I):
+    I = I // 8 * 8
+    x, w, ids, w13, w2 = _expert_case(T * 7 + K, T, H, I, E, K, dtype)
+    xd, wd, idd, w13d, w2d = _dev_case(x, w, ids, w13, w2)
+    if T * K > 2:
+        idd[T - 1, K - 1] = -1
+    whole = run_experts(xd, wd, idd, w13d, w2d)
+    for t in range(T):
+        one = run_experts(xd[t:t + 1], wd[t:t + 1].contiguous(), idd[t:t + 1].contiguous(), w13d,
+                          w2d)
+        assert torch.equal(one[0], whole[t]), t
+
+
 def test_experts_absent_slot_contributes_zero():
     x, w, ids, w13, w2 = _expert_case(5, 1, 512, 256, 8, 2, torch.float32)
     slots = torch.tensor(ids, dtype=torch.int32)

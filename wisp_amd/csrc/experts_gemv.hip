@@ -186,6 +186,56 @@ __global__ __launch_bounds__(256) void w13_silu_kernel(const T* __restrict__ x, 
                         w13_stride, act, lane);
 }
 
+// Kernel A for calls whose tokens may share experts: of the pairs with one
+// slot, the first one's block computes them all from one read of its rows,
+// and the others' blocks end at once.  P = T * K <= kSharedPairs; each wave
+// finds its slot's pairs by ballot over the call's slots.  Every pair's
+// arithmetic is w13_wave's.  What bounds it is the stream of the distinct
+// experts' rows.  Measured, every pair's own read against this (us per call,
+// w2 and the router included): Qwen3 40.6 -> 39.3 / 51.2 -> 49.0 / 81.7 ->
+// 73.8 / 111.9 -> 96.5 / 132.1 -> 109.9 at 3 / 4 / 7 / 10 / 12 tokens, Mixtral
+// 211 -> 204 / 310 -> 278 at 2 / 3; at two Qwen3 tokens, which share one
+// expert in 16, 30.3 -> 30.2.
+template <typename T, int CH, bool FULL>
+__global__ __launch_bounds__(256) void w13_shared_kernel(const T* __restrict__ x, int H, int I,
+                                                          int K, int P,
+                                                          const int32_t* __restrict__ slots,
+                                                          const T* __restrict__ w13,
+                                                          size_t w13_stride,
+                                                          T* __restrict__ act, int nslots) {
+  constexpr int V = Vec<T>::N;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int pair = blockIdx.y;
+  const int i = blockIdx.x * 4 + wave;
+  const int a0 = slots[min(lane, P - 1)], a1 = slots[min(64 + lane, P - 1)];
+  const int nch = H / V;
+  uint4 xv[CH], wg[CH], wu[CH];
+  load_row<T, CH, FULL, false>(x + (size_t)(pair / K) * H, nch, lane, xv);
+  if (i >= I) return;
+  const int s = pair < 64 ? __builtin_amdgcn_readlane(a0, pair)
+                          : __builtin_amdgcn_readlane(a1, pair - 64);
+  if ((unsigned)s >= (unsigned)nslots) {  // as a slot of -1
+    if (lane == 0) store_elem(act + (size_t)pair * I + i, 0.f);
+    return;
+  }
+  uint64_t b0 = __ballot(lane < P && a0 == s), b1 = __ballot(64 + lane < P && a1 == s);
+  if ((b0 ? __builtin_ctzll(b0) : 64 + __builtin_ctzll(b1)) != pair) return;
+  const T* W = w13 + (size_t)s * w13_stride;
+  load_row<T, CH, FULL, true>(W + (size_t)i * H, nch, lane, wg);
+  load_row<T, CH, FULL, true>(W + (size_t)(I + i) * H, nch, lane, wu);
+  for (int p = pair;;) {
+    const float v = swiglu_rows<T, CH, uint4>(wg, wu, xv);
+    if (lane == 0) store_elem(act + (size_t)p * I + i, v);
+    if (b0)
+      b0 &= b0 - 1;
+    else
+      b1 &= b1 - 1;
+    if (!(b0 | b1)) return;
+    p = b0 ? __builtin_ctzll(b0) : 64 + __builtin_ctzll(b1);
+    load_row<T, CH, FULL, false>(x + (size_t)(p / K) * H, nch, lane, xv);
+  }
+}
+
 // ---------------------------------------------------------------------------
 // Kernel A for a resident layer's smallest calls, with the router in front:
 // block (i, pair) routes its own token (wave 0, and only as many rounds as
@@ -194,12 +244,14 @@ __global__ __launch_bounds__(256) void w13_silu_kernel(const T* __restrict__ x, 
 // has all of its choices and writes them for w2.  E <= 128, whole rows.
 // Such a call is bound by its launches: the router's took 3.8 us for one
 // wave's work.  Measured, separate launches against this one (us per call):
-// Qwen3 18.9 -> 16.5 / 30.2 -> 28.7 / 50.8 -> 49.5 / 81.5 -> 80.2 at 1 / 2 /
-// 4 / 7 tokens, the fp32 toy layer 17.1 -> 14.5; with eight chunks a lane
-// (Mixtral) 110.7 -> 110.0 at one token but 210.2 -> 210.9 at two, so there
-// only one-token calls take it.
+// Qwen3 18.9 -> 16.5 / 30.2 -> 28.7 at 1 / 2 tokens, the fp32 toy layer
+// 17.1 -> 14.5 at 1 to 8, Mixtral 110.7 -> 110.0 at one.  It reads every
+// pair's rows, so where those are a stream of their own two tokens are its
+// limit: at 3 Qwen3 tokens (151 MB) 40.2 against w13_shared_kernel's 39.3,
+// at two Mixtral tokens (939 MB) 211 against 204.
 // ---------------------------------------------------------------------------
 constexpr int kRouteW13Tokens = 8;
+constexpr double kRouteW13Bytes = 128e6;  // of the pairs' w13 rows, past one token
 
 template <typename TL>
 struct RouteArgs {
@@ -802,6 +854,15 @@ template <typename T, int CH>
 void launch_w13(const T* x, int T_, int H, int I, int K, const int32_t* slots, const T* w13,
                 size_t w13_stride, T* act, hipStream_t st, const LaunchCtl& c) {
   dim3 grid((I + 3) / 4, T_ * K);
+  if (T_ >= 2 && T_ * K <= kSharedPairs && !c.pair_filter) {
+    if (H == CH * 64 * Vec<T>::N)
+      launch_timed(w13_shared_kernel<T, CH, true>, grid, dim3(256), st, c.start, c.stop, x, H, I,
+                   K, T_ * K, slots, w13, w13_stride, act, c.nslots);
+    else
+      launch_timed(w13_shared_kernel<T, CH, false>, grid, dim3(256), st, c.start, c.stop, x, H, I,
+                   K, T_ * K, slots, w13, w13_stride, act, c.nslots);
+    return;
+  }
   if (H == CH * 64 * Vec<T>::N)
     launch_timed(w13_silu_kernel<T, CH, true>, grid, dim3(256), st, c.start, c.stop, x, H, I, K,
                  slots, w13, w13_stride, act, c.pair_filter, c.want, c.nslots);
@@ -1034,11 +1095,12 @@ int decode_w13(const PageInArgs& a, const void* x, int dtype, int logits_dtype, 
 
 // Whether route_w13 serves a resident layer's call (the router instance of
 // two logits a lane, whole rows of 1, 2, 4 or 8 chunks).
-bool route_w13_supported(int dtype, int T_, int H, int E, int K) {
+bool route_w13_supported(int dtype, int T_, int H, int I, int E, int K) {
   const int V = dtype == WISP_F32 ? 4 : 8;
   const int ch = H / V / 64;
-  return T_ >= 1 && T_ <= (ch == 8 ? 1 : kRouteW13Tokens) && E <= 128 && K <= E &&
-         H % (64 * V) == 0 && (ch == 1 || ch == 2 || ch == 4 || ch == 8) &&
+  const double bytes = (double)T_ * K * 2 * I * H * (dtype == WISP_F32 ? 4 : 2);
+  return T_ >= 1 && T_ <= kRouteW13Tokens && (T_ == 1 || bytes <= kRouteW13Bytes) && E <= 128 &&
+         K <= E && H % (64 * V) == 0 && (ch == 1 || ch == 2 || ch == 4 || ch == 8) &&
          gemv_supported(dtype, H, K);
 }
 

@@ -73,7 +73,7 @@ int launch_pager(const int32_t* ids, const void* logits, int logits_dtype, int r
 int gemv_w13(const void* x, int dtype, int T, int H, int I, int K, const int32_t* slots,
              int nslots, const void* w13, size_t w13_stride, void* act, hipStream_t st,
              hipEvent_t ev_start, hipEvent_t ev_stop, const int32_t* pair_filter, int want);
-bool route_w13_supported(int dtype, int T, int H, int E, int K);
+bool route_w13_supported(int dtype, int T, int H, int I, int E, int K);
 int route_w13(const void* logits, int logits_dtype, int E, int renorm, float* topk_w,
               int32_t* topk_ids, int64_t* forward, const void* x, int dtype, int T, int H, int I,
               int K, const void* w13, size_t w13_stride, void* act, hipStream_t st, hipEvent_t e0,
@@ -666,22 +666,25 @@ int experts(Layer& L, const void* x, int T, int K, const float* w, const int32_t
 
 // Whether a call that auto_algo gives the decode kernels is faster on the
 // grouped ones because its tokens share experts.  Uniform routing over E
-// experts makes T tokens meet D = E (1 - (1 - K / E)^T) distinct ones; the
-// decode kernels stream T * K experts' weights, the grouped ones D and three
-// small launches more.  Measured, T * K / D and decode against grouped (us):
-// bf16 Mixtral (8 experts, top-2) 1.14 / 1.30 / 1.46 / 1.82 / 2.22 at 2 / 3 /
-// 4 / 6 / 8 tokens, 211 / 312 / 409 / 613 / 821 against 230 / 292 / 309 /
-// 363 / 405; bf16 Qwen3 (128, top-8) 1.39 / 1.47 at 12 / 14 tokens, 133 / 153
-// against 140 / 144.  Block-FP8 Qwen3, 1.24 / 1.39 / 1.55 at 8 / 12 / 16
-// tokens: 90 / 107 / 125 against 94 / 96 / 109.  Like auto_algo it depends on
-// the shape and the token count alone.
+// experts makes T tokens meet D = E (1 - (1 - K / E)^T) distinct ones.  The
+// bf16 decode kernels read w13 once per distinct expert (up to kSharedPairs
+// pairs, else per pair) and w2 per pair, the grouped ones everything once for
+// three small launches more, which pays from about 220 MB on.  Measured,
+// excess bytes and decode against grouped (us): Mixtral (8 experts, top-2)
+// 60 / 160 / 296 / 456 MB at 2 / 3 / 4 / 5 tokens, 198 / 281 / 348 / 426
+// against 230 / 293 / 309 / 363; Qwen3 (128, top-8) 73 / 98 / 145 MB at 12 /
+// 13 / 16 tokens, 113 / 120 / 139 against 140 / 142 / 147.  Block-FP8 goes by
+// T * K / D from 1.3 on: Qwen3, 1.24 / 1.39 / 1.55 at 8 / 12 / 16 tokens, 90 /
+// 107 / 125 against 94 / 96 / 109.  Like auto_algo it depends on the shape and
+// the token count alone.
 bool shares_experts(int dtype, int H, int I, int E, int T, int K) {
   if (dtype == WISP_F32 || T < 2 || K > E) return false;
-  if (dtype == WISP_BF16 && !mfma_supported(H, I)) return false;
   double absent = 1.0;
   for (int t = 0; t < T && absent > 1e-6; ++t) absent *= 1.0 - (double)K / E;
-  const double ratio = dtype == WISP_BF16 ? 1.45 : 1.3;
-  return (double)T * K >= ratio * E * (1.0 - absent);
+  const double pairs = (double)T * K, distinct = E * (1.0 - absent);
+  if (dtype == WISP_FP8_E4M3) return pairs >= 1.3 * distinct;
+  return mfma_supported(H, I) &&
+         (pairs - distinct) * (pairs <= kSharedPairs ? 1 : 3) * 2.0 * H * I >= 220e6;
 }
 
 // The expert algorithm of a layer call (-1: the request does not cover it).
@@ -1070,7 +1073,7 @@ extern "C" int wisp_layer_forward(void* handle, const void* x, const void* logit
   if (d.mode == WISP_MODE_RESIDENT) {
     if (a == WISP_ALGO_GEMV && !L->fp8 && logits &&
         (logits_dtype == WISP_F32 || logits_dtype == WISP_BF16) && ws->topk_w && ws->topk_ids &&
-        route_w13_supported(d.dtype, T, d.hidden, d.num_experts, K)) {
+        route_w13_supported(d.dtype, T, d.hidden, d.inter, d.num_experts, K)) {
       // [route + w13] [w2]
       ProfLaunch* p = prof_begin(*L, 0);
       if (p) L->prof_w13_calls += 1;
