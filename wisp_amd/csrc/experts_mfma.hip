@@ -633,7 +633,8 @@ __attribute__((amdgpu_waves_per_eu(Sh::kWaves / 4, Sh::kWaves / 4))) void mfma_t
 // 4. combine: out[t, h] = bf16(sum_k w[t,k] * y[(t,k), h]), k ascending,
 // skipping pairs without a slot (their y rows are never written: selected
 // out, not multiplied by zero).  8 columns per thread, every k's slot,
-// weight and y loads issued before the sums.  grid = (ceil(H / 2048), T).
+// weight and y loads issued before the sums; y is read once, non-temporally
+// (118 -> 100 us for the 537 MB of an 8192-token Qwen3 call).  grid = (ceil(H / 2048), T).
 // ---------------------------------------------------------------------------
 constexpr int kCombineK = 16;  // top-k handled with all loads up front; more loop
 
@@ -659,8 +660,8 @@ __global__ __launch_bounds__(256) void combine_kernel(const float* __restrict__ 
         ok[k] = sl >= 0 && sl < nslots;
         w[k] = topk_w[p];
         const f32x4* yr = reinterpret_cast<const f32x4*>(y + (size_t)p * H + h);
-        lo[k] = yr[0];
-        hi[k] = yr[1];
+        lo[k] = __builtin_nontemporal_load(yr);
+        hi[k] = __builtin_nontemporal_load(yr + 1);
       }
     }
 #pragma unroll
