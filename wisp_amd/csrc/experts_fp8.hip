@@ -1807,7 +1807,8 @@ __attribute__((amdgpu_waves_per_eu(Sh::kWaves / 4, Sh::kWaves / 4))) void fp8_ti
     L.lt[u] = dma::swz(L.wt * 16 + (L.lane & 15), cb);
   }
   L.tokens = {a.A, (uint32_t)a.rows * (uint32_t)L.Kdim};
-  static_assert(Sh::kWaves * tile::kRowsPerCopy == 64 && Sh::NG % 4 == 0, "weight_row(64 i + r) is weight_row(64 i) + weight_row(r) for r < 64");
+  // weight_row(64 i + r) is weight_row(64 i) + weight_row(r) for r < 64
+  static_assert(Sh::kWaves * tile::kRowsPerCopy == 64 && Sh::NG % 4 == 0, "rows of a copy step");
   L.woff = (uint32_t)L.weight_row(L.copy_row(0)) * (uint32_t)L.Kdim +
            (((L.lane % dma::kLanesPerRow) ^ (L.copy_row(0) & 7)) << 4);
 #pragma unroll

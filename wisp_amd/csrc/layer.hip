@@ -137,10 +137,13 @@ bool mfma_supported(int H, int I);
 bool gemv_supported(int dtype, int H, int K);
 
 // Calls of at least this many tokens run the bf16 experts on the MFMA grouped
-// GEMM; fewer run the GEMV kernels, which stream each routed expert once per
-// token and win while the tokens of a call share few experts.  Measured on
-// MI355X at the Qwen3 shape with uniform routing (resident, us per call):
-// GEMV 136 / 158 / 178 and MFMA 141 / 147 / 153 at 12 / 14 / 16 tokens.
+// GEMM; fewer run the GEMV kernels, unless their tokens share large experts
+// (shares_experts).  Measured on MI355X at the Qwen3 shape with uniform routing
+// (resident, us per call): GEMV 113 / 127 / 139 and MFMA 140 / 144 / 147 at 12 /
+// 14 / 16 tokens (184 and 148 at 17, past kSharedPairs).  From 14 tokens on
+// the paged calls decide: paged and resident calls of one size take one
+// family, and only the grouped GEMM's go by phases, which saves a call whose
+// experts do not fit most of its copies (milliseconds).
 constexpr int kMfmaMinTokens = 14;
 // The block-FP8 grouped path takes over from its decode kernels from here.
 constexpr int kFp8GroupedMinTokens = 16;
