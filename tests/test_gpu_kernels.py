@@ -426,6 +426,42 @@ def test_experts_mfma_tiles_equal_the_small_blocks(H, I, reps):
     assert rel_err(whole[pick.to(DEV)], ref) < 4e-3
 
 
+# Every 64 columns of act start their k loop at a 64-column place of their own,
+# whatever kernel computes them: the 64-token blocks (40 pairs), tiles of 192
+# tokens (few slots) and of 256 (more tiles than CUs).  I 256: the halves of a
+# 128-column tile start 2 of 8 chunks apart; 768: 2 or 3 of 32; 1536: 0 or 1 of 8.
+@pytest.mark.parametrize("H,I,E,per", [(512, 256, 2, 20), (512, 256, 2, 100), (2048, 768, 2, 100),
+                                       (512, 1536, 24, 64), (4096, 256, 3, 300),
+                                       (512, 768, 48, 130)])
+def test_w13_k_order_of_every_64_columns(H, I, E, per):
+    """Gate rows hold one value per 32-column step: 2^25 at the first step of
+    the k order, -2^25 at a later one, 1 elsewhere.  A 1 added to 2^25 is
+    lost, so the sum counts the steps after the later one."""
+    rng = np.random.default_rng(H + I + E)
+    steps, panels = H // 32, I // 64
+    gate = np.zeros((E, I, H), dtype=np.float32)
+    vals = np.ones((E, I, steps), dtype=np.float32)
+    start = 2 * (np.arange(I) // 64 * (H // 64) // panels)  # the first step of a column's order
+    after = rng.integers(1, steps, (E, I))  # where in the order -2^25 comes
+    vals[:, np.arange(I), start] = 2.0 ** 25
+    np.put_along_axis(vals, ((start + after) % steps)[..., None], -(2.0 ** 25), 2)
+    gate[:, :, ::32] = vals
+    want = steps - 1 - after
+    w13 = torch.zeros((E, 2 * I, H), dtype=torch.bfloat16)
+    w13[:, :I] = torch.from_numpy(gate)
+    w13[:, I:, 0] = 1.0
+    pick = np.arange(H) * I // H if H < I else np.arange(H) % I
+    w2 = torch.zeros((E, H, I), dtype=torch.bfloat16)
+    w2[:, torch.arange(H), torch.from_numpy(pick)] = 1.0  # out columns show act columns
+    ids = np.repeat(np.arange(E), per).astype(np.int32)[:, None]
+    x = torch.ones((E * per, H), dtype=torch.bfloat16)
+    out = run_experts(*_dev_case(x, np.ones((E * per, 1), dtype=np.float32), ids, w13, w2),
+                      algo=MFMA).float().cpu()
+    g = torch.from_numpy(want[:, pick]).double()
+    # silu of a whole number, rounded to bf16: neighbours are further apart
+    assert (out.view(E, per, H) - (g * torch.sigmoid(g))[:, None]).abs().max() < 0.3
+
+
 def test_experts_mfma_absent_slot_contributes_zero():
     x, w, ids, w13, w2 = _expert_case(6, 20, 512, 256, 8, 2, torch.bfloat16)
     slots = torch.tensor(ids, dtype=torch.int32)

@@ -144,9 +144,9 @@ __global__ __launch_bounds__(64 * NW) void gather_kernel(const int32_t* __restri
 // Qwen3 w13 tensor in this order, non-temporal loads: 6.27 TB/s on MI355X).
 // Starting each group of panels at its own multiple of 64 columns, evenly
 // spread over the row, and wrapping around gives 6.99 TB/s.  The start depends
-// only on the output column's group (128 columns of I in w13, 256 of H in w2:
-// what the widest block covers), never on the slot, so an output's dot-product
-// order is the same for any slot placement, token grouping or block size.
+// only on the output column's group (64 columns of I in w13, 256 of H in w2),
+// never on the slot, so an output's dot-product order is the same for any slot
+// placement, token grouping or block size.
 __device__ inline int k_rotation(unsigned group, unsigned groups, int Kdim) {
   return (int)(group * (unsigned)(Kdim / 64) / groups) * 64;
 }
@@ -273,7 +273,7 @@ __global__ __launch_bounds__(256) void mfma_w13_dma_kernel(
     wrow[i] = reinterpret_cast<const unsigned char*>(
         W + (size_t)(r < 16 ? i0 + r : I + i0 + r - 16) * H);
   }
-  const int rot = k_rotation(blockIdx.x / 2, gridDim.x / 2, H);
+  const int rot = k_rotation(blockIdx.x, gridDim.x, H);
   for (int m0 = 0; m0 < M; m0 += dma::kTokRows) {
     const int mrows = min(M - m0, dma::kTokRows);
     if (m0 > 0) held = dma::list_entries(list, m0, P);
@@ -351,6 +351,13 @@ __global__ __launch_bounds__(256) void mfma_w2_dma_kernel(
 // touching the lines three chunks ahead (557 + 361: the loads of a CU
 // return in order), 320-token tiles (492 + 335, registers spill), 128 x 128
 // tiles with two blocks per CU (545 + 351), no k rotation (447 + 329).
+// These are figures of tiles whose halves started their k loops together.
+// They start apart, each at its 64 columns' own place, because the 64-token
+// blocks do: 2 or 3 of 32 chunks at this shape, in which one half of the waves
+// has no products and its rows are not copied.  That costs w13 4 % here
+// (rocprofv3: 505 -> 525 us) and 2 % at a 1000-token Mixtral chunk (585 -> 596).
+// Peeling those steps off the loop, or the other assignment of waves to halves
+// (both waves of a SIMD to one), changed nothing.
 // ---------------------------------------------------------------------------
 struct TileArgs {
   const uint16_t* A;  // token matrix: x (w13) or act (w2)
@@ -408,7 +415,7 @@ struct TileLoop {
     if (!kW13) return r;
     return r / (2 * half) * half + r % half + (r % (2 * half) < half ? 0 : a.I);
   }
-  // The pairs behind this lane's token copies and the token row it touches.
+  // The pairs behind this lane's token copies.
   struct Pairs {
     int copy[Sh::kTCopies];
   };
@@ -431,11 +438,18 @@ struct TileLoop {
                    (((lane % dma::kLanesPerRow) ^ (copy_row(i) & 7)) << 4);
     constexpr int per = tile::kRowsPerCopy * Sh::kWaves, step = 16 * Sh::WT;
     s->tc = ((w.mrows + step - 1) / step * step + per - 1) / per;
-    s->rot = k_rotation(w.panel * Sh::kRows / 256, N / 256, Kdim) * 2;
+    // a w13 panel's two halves (64 columns each) start their k loops apart
+    const int half0 = kW13 ? 2 * w.panel : w.panel, halves = kW13 ? 2 * npanels : npanels;
+    s->rot = k_rotation(half0, halves, Kdim) * 2;
+    s->lag = kW13 ? (k_rotation(half0 + 1, halves, Kdim) * 2 - s->rot) / tile::kRowBytes : 0;
   }
   __device__ __attribute__((always_inline)) void issue(unsigned char* stage,
                                                        const tile::Source<Sh>& s, int c) const {
-    tile::copies<Sh>(stage, s, woff, wstep, tokens, wave, tile::chunk_byte(c, s.rot, Kdim * 2));
+    // the first half's rows are not needed past its last chunk, nor the
+    // second's before its first
+    tile::copies<Sh>(stage, s, woff, wstep, tokens, wave, tile::chunk_byte(c, s.rot, Kdim * 2),
+                     kW13 && c >= chunks ? Sh::kWCopies / 2 : 0,
+                     kW13 && c < s.lag ? Sh::kWCopies / 2 : Sh::kWCopies);
   }
   template <int NT>
   __device__ __attribute__((always_inline)) void read_t(const unsigned char* stage, int u, int i,
@@ -461,16 +475,19 @@ struct TileLoop {
   // One chunk, from stage `rds`, with the next chunk's copies into `wrs`
   // (distinct stages, see dma::step): fragment by fragment in the order of
   // the matrix instructions, each read kAhead groups before its use.  The
-  // last kLeft groups of the chunk before (unless kFirst) cover the first
-  // reads, and this chunk's are left for the next call: all its fragments
-  // are then in registers, so that its stage can be overwritten.
-  template <int NT, bool kFirst>
+  // last kLeft groups of the chunk before (zeros before a tile's first) cover
+  // the first reads, and this chunk's are left for the next call: all its
+  // fragments are then in registers, so that its stage can be overwritten.
+  // A wave that is not `active` has no products in this chunk.
+  template <int NT>
   __device__ __attribute__((always_inline)) void chunk(unsigned char* __restrict__ wrs,
                                                        const unsigned char* __restrict__ rds,
                                                        const tile::Source<Sh>& cs, int cc,
-                                                       Frags<NT>& f, f32x4 (&acc)[NG][NT]) const {
+                                                       bool active, Frags<NT>& f,
+                                                       f32x4 (&acc)[NG][NT]) const {
     if (cc >= 0) issue(wrs, cs, cc);
     __builtin_amdgcn_sched_barrier(0);
+    if (!active) return;
     // positions -kLeft .. 2 NG - kLeft - 1; before position n: token
     // fragments of the first k-step, then weight fragment n + kAhead
 #pragma unroll
@@ -483,10 +500,7 @@ struct TileLoop {
         for (int i = n * NT / (NG - 1); i < (n + 1) * NT / (NG - 1); ++i)
           read_t<NT>(rds, 1, i, f);
       }
-      if (n >= 0)
-        mma<NT>(n, f, acc);
-      else if (!kFirst)
-        mma<NT>(2 * NG + n, f, acc);
+      mma<NT>(n >= 0 ? n : 2 * NG + n, f, acc);
       __builtin_amdgcn_sched_barrier(0);
     }
   }
@@ -509,16 +523,19 @@ struct TileLoop {
     dma::wait_vm<N * kStores>();
     dma::lds_barrier();
   }
-  template <int NT, bool kFirst = false>
+  template <int NT>
   __device__ __attribute__((always_inline)) void next_chunk(const tile::Source<Sh>& cs, int cc,
-                                                            Frags<NT>& f, f32x4 (&acc)[NG][NT]) {
-    chunk<NT, kFirst>(smem + (~q & 1) * Sh::kStage, smem + (q & 1) * Sh::kStage, cs, cc, f,
-                      acc);
+                                                            bool active, Frags<NT>& f,
+                                                            f32x4 (&acc)[NG][NT]) {
+    chunk<NT>(smem + (~q & 1) * Sh::kStage, smem + (q & 1) * Sh::kStage, cs, cc, active, f, acc);
     ++q;
   }
 
-  // One tile.  On entry the copies of its first chunk and the touches of the
-  // next two are issued; on return those of the next tile's are, if any.
+  // One tile.  On entry the copies of its first chunk are issued; on return
+  // those of the next tile's are, if any.  Its chunks + lag chunks start at
+  // the first half's k rotation; the waves of the second half pass the first
+  // `lag` of them, where their own rotation has not begun, and those of the
+  // first half the last `lag`, which are past their end.
   template <int NT>
   __device__ __attribute__((always_inline)) void run(tile::Work& w, tile::Source<Sh>& src,
                                                      bool* more) {
@@ -528,6 +545,10 @@ struct TileLoop {
 #pragma unroll
       for (int t = 0; t < NT; ++t) acc[g][t] = f32x4{0.f, 0.f, 0.f, 0.f};
     Frags<NT> f;
+#pragma unroll
+    for (int n = 2 * NG - kLeft; n < 2 * NG; ++n) f.w[n % kRing] = bf16x8{};
+#pragma unroll
+    for (int t = 0; t < NT; ++t) f.t[1][t] = bf16x8{};
     int pr[NT];
     Pairs np;
     tile::Work nw;
@@ -540,14 +561,14 @@ struct TileLoop {
 #pragma unroll
     for (int t = 0; t < NT; ++t)
       pr[t] = list(w)[min((t * Sh::WT + wt) * 16 + (lane & 15), w.mrows - 1)];
-    next_chunk<NT, true>(src, 1, f, acc);
-    wait();
-    if (next) source(nw, np, &ns);
-    for (int c = 1; c < chunks - 1; ++c) {
-      next_chunk<NT>(src, c + 1, f, acc);
+    const int lag = kW13 ? __builtin_amdgcn_readfirstlane(src.lag) : 0;
+    const int begin = wr < Sh::WR / 2 ? 0 : lag, steps = chunks + lag;
+    for (int c = 0; c < steps - 1; ++c) {
+      next_chunk<NT>(src, c + 1, !kW13 || (c >= begin && c < begin + chunks), f, acc);
       wait();
     }
-    next_chunk<NT>(ns, next ? 0 : -1, f, acc);
+    if (next) source(nw, np, &ns);
+    next_chunk<NT>(ns, next ? 0 : -1, begin == lag, f, acc);
 #pragma unroll
     for (int n = 2 * NG - kLeft; n < 2 * NG; ++n) mma<NT>(n, f, acc);
 #pragma unroll
@@ -588,8 +609,10 @@ __attribute__((amdgpu_waves_per_eu(Sh::kWaves / 4, Sh::kWaves / 4))) void mfma_t
   L.chunks = L.Kdim * 2 / tile::kRowBytes;
   L.wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   L.lane = threadIdx.x & 63;
-  L.wr = L.wave % Sh::WR;
-  L.wt = L.wave / Sh::WR;
+  // (waves w and w + 4 share a SIMD: one of each half of the rows)
+  static_assert(Sh::kWaves == 8 && Sh::WR % 2 == 0, "halves of the rows over the SIMDs");
+  L.wr = L.wave / Sh::WT;
+  L.wt = L.wave % Sh::WT;
 #pragma unroll
   for (int u = 0; u < 2; ++u) {
     L.lw[u] = dma::swz(L.wr * Sh::NG * 16 + (L.lane & 15), u * 4 + (L.lane >> 4));

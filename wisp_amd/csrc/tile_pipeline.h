@@ -144,13 +144,14 @@ __device__ __attribute__((always_inline)) inline void copy16(const Range& r, uin
 // Where a tile's rows are: the range its weight rows lie in, the byte of the
 // row the chunk sequence starts at, and this lane's offset of each of its
 // wave's token copies (copy i of wave w covers rows
-// [(i * kWaves + w) * kRowsPerCopy, +kRowsPerCopy)) and of the row it touches.
+// [(i * kWaves + w) * kRowsPerCopy, +kRowsPerCopy)).
 template <typename Sh>
 struct Source {
   Range w;
   uint32_t toff[Sh::kTCopies];
   int tc;  // token copies each wave makes
   int rot;
+  int lag;  // chunks by which the second half of the weight rows starts later
 };
 
 __device__ inline int chunk_byte(int c, int rot, int row_bytes) {
@@ -158,15 +159,18 @@ __device__ inline int chunk_byte(int c, int rot, int row_bytes) {
   return o >= row_bytes ? o - row_bytes : o;
 }
 
+// One chunk's copies: weight copies [w0, w1) of each wave, and its tokens'.
 template <typename Sh>
 __device__ __attribute__((always_inline)) inline void copies(
     unsigned char* st, const Source<Sh>& src, uint32_t woff,
-    const uint32_t (&wstep)[Sh::kWCopies], const Range& tokens, int wave, int o) {
+    const uint32_t (&wstep)[Sh::kWCopies], const Range& tokens, int wave, int o, int w0 = 0,
+    int w1 = Sh::kWCopies) {
   const Range wr = scalar(src.w), tr = scalar(tokens);
   o = __builtin_amdgcn_readfirstlane(o);
 #pragma unroll
   for (int i = 0; i < Sh::kWCopies; ++i)
-    copy16(wr, woff, o + (int)wstep[i], st + (i * Sh::kWaves + wave) * 1024);
+    if (i >= w0 && i < w1)
+      copy16(wr, woff, o + (int)wstep[i], st + (i * Sh::kWaves + wave) * 1024);
 #pragma unroll
   for (int i = 0; i < Sh::kTCopies; ++i)
     if (i < src.tc)
