@@ -515,8 +515,10 @@ def test_install_wisp_fp8_standin_layer_matches_resident():
     E, H, I, K, block = 16, 512, 256, 4, (128, 128)
     _, w13, w2, s13, s2 = _experts(E, H, I, block, seed=13)
     g = torch.Generator().manual_seed(14)
-    x = torch.randn((3, H), generator=g).to(torch.bfloat16).to(DEV)
-    lg = torch.randn((3, E), generator=g).to(DEV)
+    # few tokens, and more whose tokens share experts, up to the grouped path
+    calls = [(torch.randn((T, H), generator=g).to(torch.bfloat16).to(DEV),
+              torch.randn((T, E), generator=g).to(DEV)) for T in (3, 4, 12, 15, 16)]
+    x, lg = calls[0]
     names = ("create_weights", "process_weights_after_loading", "apply")
     saved = {n: Fp8MoEMethod.__dict__[n] for n in names}
     was_patched = getattr(Fp8MoEMethod, f8m._PATCHED_FLAG, False)
@@ -528,7 +530,7 @@ def test_install_wisp_fp8_standin_layer_matches_resident():
         plain = Fp8FusedMoE(E, K, H, I, block)  # unpatched: every expert on the GPU
         plain.load_weights(w13, w2, s13, s2)
         plain.process_weights_after_loading()
-        ref = plain(x, lg)
+        refs = [plain(*c) for c in calls]
         assert f8m.install_wisp_fp8() and f8m.is_fp8_installed()
         assert not f8m.install_wisp_fp8()  # idempotent
         paged = Fp8FusedMoE(E, K, H, I, block)
@@ -538,9 +540,10 @@ def test_install_wisp_fp8_standin_layer_matches_resident():
         st = paged._wisp_fp8_state
         assert st.cap_experts == min(E, 24) and st.pagein_engine == "kernel"
         assert paged.w13_weight.numel() == 0  # device placeholder
-        out = paged(x, lg)
-        torch.cuda.synchronize()
-        assert torch.equal(out.view(torch.int16), ref.view(torch.int16))
+        for c, ref in zip(calls, refs):
+            out = paged(*c)
+            torch.cuda.synchronize()
+            assert torch.equal(out.view(torch.int16), ref.view(torch.int16)), c[0].shape
         with pytest.raises(NotImplementedError):
             paged.quant_method.apply(paged, x, lg, K, True, expert_map=torch.zeros(E))
     finally:

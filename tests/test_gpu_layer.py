@@ -9,7 +9,7 @@ from oracle.pager import PagerOracle
 from tests._util import fixture_matches, load_golden, oracle_trace_matches
 from wisp_amd import _lib
 from wisp_amd import workloads as W
-from wisp.integrations.vllm.fused_moe import WispMoEState
+from wisp.integrations.vllm.fused_moe import WispMoEState, _route_and_experts
 from wisp_amd.record import parse_record
 
 pytestmark = pytest.mark.gpu
@@ -712,3 +712,27 @@ def test_resident_calls_routed_in_the_w13_launch(dtype, H, I, E, K, tokens, logi
                 assert torch.equal(ids, ir) and torch.equal(w, wr), (T, renorm)
                 assert torch.equal(bits(out), bits(ref)), (T, renorm)
     assert st.stats_forward == calls
+
+
+def test_few_token_calls_of_large_experts_have_one_family():
+    """Calls whose few tokens share large experts (2 to 13 tokens over 4
+    experts of 100 MB, and 14, the grouped GEMM): resident, paged in token
+    groups and copy mode's entry point give the same bytes."""
+    H, I, E, K = 4096, 4096, 4, 2
+    g = torch.Generator(device=DEV).manual_seed(9)
+    w13 = torch.empty((E, 2 * I, H), dtype=torch.bfloat16, pin_memory=True)
+    w2 = torch.empty((E, H, I), dtype=torch.bfloat16, pin_memory=True)
+    for w in (w13, w2):
+        w.copy_(torch.randn(w.shape, generator=g, device=DEV, dtype=torch.bfloat16) * 0.02)
+    res = WispMoEState(w13, w2, E, "resident", DEV, 0)
+    res.prime_identity()
+    paged = WispMoEState(w13, w2, 2, "paged", DEV, 0)
+    w13d, w2d = w13.to(DEV), w2.to(DEV)
+    for T in (2, 3, 5, 6, 13, 14):
+        x = torch.randn((T, H), generator=g, device=DEV, dtype=torch.bfloat16)
+        lg = torch.randn((T, E), generator=g, device=DEV)
+        a, b = res.forward(x, lg, K, True), paged.forward(x, lg, K, True)
+        c = _route_and_experts(x, lg, K, True, w13d, w2d)
+        torch.cuda.synchronize()
+        assert torch.equal(bits(a), bits(b)), T
+        assert torch.equal(bits(a), bits(c)), T

@@ -25,8 +25,8 @@ constexpr int kFusedRouteTokens = 8;
 // Routed experts per token the decode GEMV pair handles (its w2 kernel runs
 // one wave per expert in one block and keeps their partial sums in LDS).
 constexpr int kGemvMaxTopK = 16;
-// (token, k) pairs of a call up to which the decode w13 kernel reads an
-// expert's rows once for all of them (two slots a lane).
+// (token, k) pairs of a call up to which the decode kernels read an expert's
+// rows once for all of them (two slots a lane).
 constexpr int kSharedPairs = 128;
 
 // Per-layer counters kept on the device, in this order.

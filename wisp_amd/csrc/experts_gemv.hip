@@ -836,6 +836,129 @@ __global__ __launch_bounds__(1024) void w2_combine_kernel(const T* __restrict__ 
   }
 }
 
+// Kernel B for calls whose tokens may share experts, with long rows (more
+// than 4 chunks a lane): block = RPH rows of W2 for all the call's tokens.  Its
+// waves take the call's distinct slots in turn; a slot's RPH rows are read
+// once for its pairs, kSharedAtOnce at a time (from L2 for the next ones, so
+// only the last read of a row is non-temporal).  Every pair's dot product and every token's sum are
+// w2_combine_kernel's, in the same order.  P = T * K <= kSharedPairs.
+// grid = ceil(H / RPH).
+// What bounds it is the stream of the distinct experts' rows, then (from
+// about 8 tokens of 8 experts) the FMAs.  Measured at the Mixtral shape, every
+// pair's own read against this (us per call, w13 and the router included):
+// 208 -> 199 / 283 -> 260 / 357 -> 311 / 488 -> 394 / 717 -> 507 / 881 -> 586
+// at 2 / 3 / 4 / 6 / 10 / 13 tokens.  At 6 tokens w2 alone takes 131 us; with 2
+// rows a wave 152, with 1 row 188 (every wave reads the act rows again), rows
+// read with the default policy 144, two pairs at a time 165, eight rows 141.
+constexpr int kSharedAtOnce = 4;
+constexpr int kSharedWaves = 4;
+
+template <typename T, int RPH>
+__global__ __launch_bounds__(64 * kSharedWaves) void w2_shared_kernel(
+    const T* __restrict__ act, int H, int I, int K, int P, const float* __restrict__ topk_w,
+    const int32_t* __restrict__ slots, const T* __restrict__ w2, size_t w2_stride,
+    T* __restrict__ out, int nslots) {
+  constexpr int V = Vec<T>::N;
+  __shared__ float part[kSharedPairs][RPH];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int h0 = blockIdx.x * RPH, nch = I / V;
+  // pairs lane and 64 + lane; a slot outside [0, nslots) reads no expert
+  const int a0 = lane < P ? slots[lane] : -1, a1 = 64 + lane < P ? slots[64 + lane] : -1;
+  const bool ok0 = (unsigned)a0 < (unsigned)nslots, ok1 = (unsigned)a1 < (unsigned)nslots;
+  // the RPH dot products of one slot's rows with the act rows of N pairs;
+  // `last`: the rows are not read again
+  auto dots = [&](auto n, auto last, const T* const (&wrow)[RPH], const int (&p)[kSharedAtOnce]) {
+    constexpr int N = decltype(n)::value;
+    float d[N][RPH];
+    const T* arow[N];
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      arow[j] = act + (size_t)p[j] * I;
+#pragma unroll
+      for (int r = 0; r < RPH; ++r) d[j][r] = 0.f;
+    }
+#pragma unroll 1
+    for (int ch = lane; ch < nch; ch += 64) {
+      uint4 wv[RPH], av[N];
+#pragma unroll
+      for (int r = 0; r < RPH; ++r)
+        wv[r] = last ? ld16_stream(wrow[r] + (size_t)ch * V) : ld16(wrow[r] + (size_t)ch * V);
+#pragma unroll
+      for (int j = 0; j < N; ++j) av[j] = ld16(arow[j] + (size_t)ch * V);
+#pragma unroll
+      for (int r = 0; r < RPH; ++r) {
+        float wf[V];
+        Vec<T>::unpack(wv[r], wf);
+#pragma unroll
+        for (int j = 0; j < N; ++j) {
+          float af[V];
+          Vec<T>::unpack(av[j], af);
+#pragma unroll
+          for (int q = 0; q < V; ++q) d[j][r] = fmaf(wf[q], af[q], d[j][r]);
+        }
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < N; ++j)
+#pragma unroll
+      for (int r = 0; r < RPH; ++r) {
+        const float v = wave_sum_f32(d[j][r]);
+        if (lane == 0) part[p[j]][r] = v;
+      }
+  };
+  uint64_t b0 = __ballot(ok0), b1 = __ballot(ok1);
+  for (int n = 0; b0 | b1; ++n) {
+    const int s = b0 ? __builtin_amdgcn_readlane(a0, __builtin_ctzll(b0))
+                     : __builtin_amdgcn_readlane(a1, __builtin_ctzll(b1));
+    uint64_t m0 = __ballot(ok0 && a0 == s), m1 = __ballot(ok1 && a1 == s);
+    b0 &= ~m0;
+    b1 &= ~m1;
+    if (n % kSharedWaves != wave) continue;
+    const T* wrow[RPH];
+#pragma unroll
+    for (int r = 0; r < RPH; ++r)
+      wrow[r] = w2 + (size_t)s * w2_stride + (size_t)min(h0 + r, H - 1) * I;
+    while (m0 | m1) {
+      int p[kSharedAtOnce], got = 0;
+#pragma unroll
+      for (int j = 0; j < kSharedAtOnce; ++j) {
+        p[j] = 0;
+        if (m0 | m1) {
+          p[j] = m0 ? __builtin_ctzll(m0) : 64 + __builtin_ctzll(m1);
+          if (m0)
+            m0 &= m0 - 1;
+          else
+            m1 &= m1 - 1;
+          ++got;
+        }
+      }
+      if (m0 | m1)
+        dots(std::integral_constant<int, 4>{}, std::false_type{}, wrow, p);
+      else if (got == 1)
+        dots(std::integral_constant<int, 1>{}, std::true_type{}, wrow, p);
+      else if (got == 2)
+        dots(std::integral_constant<int, 2>{}, std::true_type{}, wrow, p);
+      else if (got == 3)
+        dots(std::integral_constant<int, 3>{}, std::true_type{}, wrow, p);
+      else
+        dots(std::integral_constant<int, 4>{}, std::true_type{}, wrow, p);
+    }
+  }
+  __syncthreads();
+  for (int j = threadIdx.x; j < P / K * RPH; j += 64 * kSharedWaves) {
+    const int t = j / RPH, r = j % RPH;
+    if (h0 + r >= H) continue;
+    float acc = 0.f;
+    for (int k = 0; k < K; ++k) {
+      const int p = t * K + k;
+      const bool ok = (unsigned)slots[p] < (unsigned)nslots;
+      // a pair without an expert adds 0 * 0
+      acc = fmaf(ok ? topk_w[p] : 0.f, ok ? part[p][r] : 0.f, acc);
+    }
+    store_elem(out + (size_t)t * H + h0 + r, acc);
+  }
+}
+
 // Optional controls of a launch: kernel timing events, the pair filter of
 // the w13 kernel (run only pairs with pair_filter[p] == want) and the skip
 // word of the w2 kernel (exit when *skip_if != 0), and the w2 kernel's
@@ -1022,6 +1145,12 @@ int dispatch_w2(const T* act, int T_, int H, int I, int K, const float* w, const
       case 3: launch_w2<T, 32, 3, 2>(act, T_, H, I, K, w, slots, w2, w2_stride, out, st, c); break;
       default: launch_w2<T, 32, 4, 2>(act, T_, H, I, K, w, slots, w2, w2_stride, out, st, c); break;
     }
+  } else if (T_ >= 2 && T_ * K <= kSharedPairs && !c.skip_if) {
+    // (not the shorter rows: layers of many small experts, whose tokens share
+    // few of them below the grouped GEMM's token counts)
+    constexpr int RPH = 4;
+    launch_timed(w2_shared_kernel<T, RPH>, dim3((H + RPH - 1) / RPH), dim3(64 * kSharedWaves), st,
+                 c.start, c.stop, act, H, I, K, T_ * K, w, slots, w2, w2_stride, out, c.nslots);
   } else {
     launch_w2<T, 64, 0>(act, T_, H, I, K, w, slots, w2, w2_stride, out, st, c);
   }

@@ -137,8 +137,7 @@ bool mfma_supported(int H, int I);
 bool gemv_supported(int dtype, int H, int K);
 
 // Calls of at least this many tokens run the bf16 experts on the MFMA grouped
-// GEMM; fewer run the GEMV kernels, unless their tokens share large experts
-// (shares_experts).  Measured on MI355X at the Qwen3 shape with uniform routing
+// GEMM; fewer run the GEMV kernels.  Measured on MI355X at the Qwen3 shape with uniform routing
 // (resident, us per call): GEMV 113 / 127 / 139 and MFMA 140 / 144 / 147 at 12 /
 // 14 / 16 tokens (184 and 148 at 17, past kSharedPairs).  From 14 tokens on
 // the paged calls decide: paged and resident calls of one size take one
@@ -667,29 +666,6 @@ int experts(Layer& L, const void* x, int T, int K, const float* w, const int32_t
   return w2(L, act, T, K, w, slots, out, st, nullptr, nullptr);
 }
 
-// Whether a call that auto_algo gives the decode kernels is faster on the
-// grouped ones because its tokens share experts.  Uniform routing over E
-// experts makes T tokens meet D = E (1 - (1 - K / E)^T) distinct ones.  The
-// bf16 decode kernels read w13 once per distinct expert (up to kSharedPairs
-// pairs, else per pair) and w2 per pair, the grouped ones everything once for
-// three small launches more, which pays from about 220 MB on.  Measured,
-// excess bytes and decode against grouped (us): Mixtral (8 experts, top-2)
-// 60 / 160 / 296 / 456 MB at 2 / 3 / 4 / 5 tokens, 198 / 281 / 348 / 426
-// against 230 / 293 / 309 / 363; Qwen3 (128, top-8) 73 / 98 / 145 MB at 12 /
-// 13 / 16 tokens, 113 / 120 / 139 against 140 / 142 / 147.  Block-FP8 goes by
-// T * K / D from 1.3 on: Qwen3, 1.24 / 1.39 / 1.55 at 8 / 12 / 16 tokens, 90 /
-// 107 / 125 against 94 / 96 / 109.  Like auto_algo it depends on the shape and
-// the token count alone.
-bool shares_experts(int dtype, int H, int I, int E, int T, int K) {
-  if (dtype == WISP_F32 || T < 2 || K > E) return false;
-  double absent = 1.0;
-  for (int t = 0; t < T && absent > 1e-6; ++t) absent *= 1.0 - (double)K / E;
-  const double pairs = (double)T * K, distinct = E * (1.0 - absent);
-  if (dtype == WISP_FP8_E4M3) return pairs >= 1.3 * distinct;
-  return mfma_supported(H, I) &&
-         (pairs - distinct) * (pairs <= kSharedPairs ? 1 : 3) * 2.0 * H * I >= 220e6;
-}
-
 // The expert algorithm of a layer call (-1: the request does not cover it).
 // Decided before the pager runs, so a call the kernels cannot compute fails
 // without touching the pager state.
@@ -1053,13 +1029,7 @@ extern "C" int wisp_layer_forward(void* handle, const void* x, const void* logit
       return WISP_ERR_UNSUPPORTED;
     }
   }
-  int a = choose_algo(*L, algo, T, K);
-  // (only with a work buffer for it: callers that size theirs by auto_algo's
-  // choice keep the decode kernels)
-  if (algo == WISP_ALGO_AUTO && a == WISP_ALGO_GEMV &&
-      shares_experts(d.dtype, d.hidden, d.inter, d.num_experts, T, K) &&
-      work_ok(*L, WISP_ALGO_MFMA, T, K, ws))
-    a = WISP_ALGO_MFMA;
+  const int a = choose_algo(*L, algo, T, K);
   if (a < 0) {
     wisp_set_last_error("no expert kernel covers this call (shape, top_k or requested "
                         "algorithm)", "wisp_layer_forward");
