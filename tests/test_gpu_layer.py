@@ -736,3 +736,31 @@ def test_few_token_calls_of_large_experts_have_one_family():
         torch.cuda.synchronize()
         assert torch.equal(bits(a), bits(b)), T
         assert torch.equal(bits(a), bits(c)), T
+
+
+@pytest.mark.parametrize("engine,streams", [("kernel", "0"), ("memcpy", "0"), ("memcpy", "2")])
+@pytest.mark.parametrize("K,T", [(4, 40), (5, 41)])
+def test_calls_by_phases_keep_the_loaded_pairs(monkeypatch, engine, streams, K, T):
+    """A call of many token groups copies by phases; the workspace still holds
+    the (expert, slot) pairs that the pager loaded, in the record's order, and
+    the bytes are the resident layer's."""
+    monkeypatch.setenv("WISP_PAGEIN_ENGINE", engine)
+    monkeypatch.setenv("WISP_PAGEIN_STREAMS", streams)
+    H, I, E, cap = 512, 256, 32, 8
+    g = torch.Generator().manual_seed(K)
+    w13 = (torch.randn((E, 2 * I, H), generator=g) * 0.05).to(torch.bfloat16).pin_memory()
+    w2 = (torch.randn((E, H, I), generator=g) * 0.05).to(torch.bfloat16).pin_memory()
+    res = WispMoEState(w13, w2, E, "resident", DEV, 0)
+    res.prime_identity()
+    st = WispMoEState(w13, w2, cap, "paged", DEV, 1)
+    for _ in range(2):
+        x = torch.randn((T, H), generator=g).to(torch.bfloat16).to(DEV)
+        lg = torch.randn((T, E), generator=g).to(DEV)
+        out, ref = st.forward(x, lg, K, True), res.forward(x, lg, K, True)
+        torch.cuda.synchronize()
+        assert torch.equal(bits(out), bits(ref))
+        groups = parse_record(st.last_record.numpy(), T, K)["groups"]
+        pairs = [list(p) for gr in groups for p in gr["loaded"]]
+        # some expert is loaded again, so the call goes by phases
+        assert len({e for e, _ in pairs}) < len(pairs) <= T * K
+        assert st._ws.loads[:2 * len(pairs)].view(-1, 2).tolist() == pairs

@@ -146,12 +146,12 @@ struct StageEvents {
   hipEvent_t ev[4];
 };
 
-// Where a phase of a paged call finds its experts' weights: the slot of each
-// expert it covers, kDecided for the pager's own slots[p], kNone otherwise.
-// A kernel argument.
+// The expert whose weights a phase of a paged call finds in each slot; kNone:
+// the slot has no part in the phase; kDecided: the pairs that the pager gave
+// the slot (their expert stays in it for the whole call).  A kernel argument.
 struct PhaseTable {
   static constexpr int16_t kNone = -1, kDecided = -2;
-  int16_t slot[kMaxExperts];
+  int16_t expert[kMaxExperts];
 };
 
 // Per slot s < nslots, the ascending list of the pairs p < P with

@@ -67,7 +67,8 @@ struct WorkLayout {
 };
 
 // ---------------------------------------------------------------------------
-// 1. gather: lists[s * P + j] = j-th pair (ascending) with slots[p] == s.
+// 1. gather: lists[s * P + j] = j-th pair (ascending) with slots[p] == s, or,
+// for a phase of a paged call, of the expert that slot s holds in it.
 // grid = nslots; each iteration covers 8 consecutive pairs per thread and
 // places the matches by a block-wide exclusive prefix of the per-thread
 // counts (counts <= 8: four ballots per wave for the bits, one LDS exchange
@@ -81,24 +82,43 @@ struct WorkLayout {
 constexpr int kGatherPer = 8;
 constexpr int kGatherLong = 4096;  // pairs of one iteration of 8 waves
 
-template <int NW, bool kVec>
+struct WholeCall {};  // no phase
+struct Phase {
+  const int32_t* ids;  // the pairs' experts
+  PhaseTable t;
+};
+
+template <int NW, bool kVec, typename Ph>
 __global__ __launch_bounds__(64 * NW) void gather_kernel(const int32_t* __restrict__ slots, int P,
                                                          int32_t* __restrict__ lists,
-                                                         int32_t* __restrict__ counts) {
+                                                         int32_t* __restrict__ counts, Ph phase) {
   __shared__ int wave_total[2][NW];
   const int s = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int32_t* __restrict__ keys = slots;
+  int key = s;
+  if constexpr (std::is_same_v<Ph, Phase>) {
+    const int e = phase.t.expert[s];
+    if (e == PhaseTable::kNone) {
+      if (tid == 0) counts[s] = 0;
+      return;
+    }
+    if (e >= 0) {
+      keys = phase.ids;
+      key = e;
+    }
+  }
   int32_t* L = lists + (size_t)s * P;
   const uint64_t below = (1ull << lane) - 1ull;
   auto load = [&](int p0, int (&v)[kGatherPer]) {
     if (kVec && p0 + kGatherPer <= P) {
 #pragma unroll
       for (int q = 0; q < kGatherPer; q += 4) {
-        const int4 w = *reinterpret_cast<const int4*>(slots + p0 + q);
+        const int4 w = *reinterpret_cast<const int4*>(keys + p0 + q);
         v[q] = w.x, v[q + 1] = w.y, v[q + 2] = w.z, v[q + 3] = w.w;
       }
     } else {
 #pragma unroll
-      for (int q = 0; q < kGatherPer; ++q) v[q] = p0 + q < P ? slots[p0 + q] : -1;
+      for (int q = 0; q < kGatherPer; ++q) v[q] = p0 + q < P ? keys[p0 + q] : -1;
     }
   };
   int n = 0;  // matches before this iteration (block-uniform)
@@ -109,7 +129,7 @@ __global__ __launch_bounds__(64 * NW) void gather_kernel(const int32_t* __restri
     load(p0 + 64 * NW * kGatherPer, next);
     unsigned hit = 0;
 #pragma unroll
-    for (int q = 0; q < kGatherPer; ++q) hit |= (unsigned)(v[q] == s) << q;
+    for (int q = 0; q < kGatherPer; ++q) hit |= (unsigned)(v[q] == key) << q;
     const int c = __popc(hit);
     int pre = 0, tot = 0;
 #pragma unroll
@@ -817,21 +837,27 @@ bool tile_call(int P, int H, int I, int nslots, int spread, int T, uintptr_t add
 
 }  // namespace
 
-void launch_gather(const int32_t* slots, int P, int nslots, int32_t* lists, int32_t* counts,
-                   hipStream_t st) {
+template <typename Ph>
+static void gather(const int32_t* slots, int P, int nslots, int32_t* lists, int32_t* counts,
+                   bool vec, const Ph& phase, hipStream_t st) {
   auto go = [&](auto nw) {
     constexpr int NW = decltype(nw)::value;
-    if ((uintptr_t)slots % 16 == 0)
-      hipLaunchKernelGGL((gather_kernel<NW, true>), dim3(nslots), dim3(64 * NW), 0, st, slots, P,
-                         lists, counts);
+    if (vec)
+      hipLaunchKernelGGL((gather_kernel<NW, true, Ph>), dim3(nslots), dim3(64 * NW), 0, st, slots,
+                         P, lists, counts, phase);
     else
-      hipLaunchKernelGGL((gather_kernel<NW, false>), dim3(nslots), dim3(64 * NW), 0, st, slots, P,
-                         lists, counts);
+      hipLaunchKernelGGL((gather_kernel<NW, false, Ph>), dim3(nslots), dim3(64 * NW), 0, st, slots,
+                         P, lists, counts, phase);
   };
   if (P > kGatherLong)
     go(std::integral_constant<int, 16>{});
   else
     go(std::integral_constant<int, 8>{});
+}
+
+void launch_gather(const int32_t* slots, int P, int nslots, int32_t* lists, int32_t* counts,
+                   hipStream_t st) {
+  gather(slots, P, nslots, lists, counts, (uintptr_t)slots % 16 == 0, WholeCall{}, st);
 }
 
 int experts_mfma_combine(int T, int H, int K, const float* topk_w, const int32_t* slots,
@@ -851,11 +877,12 @@ namespace {
 
 // The pair lists, w13 and w2 of a call's pairs with a slot in [0, nslots):
 // their fp32 rows of y in the work buffer.  `spread`: the number of experts
-// the call's pairs spread over, for the choice of kernels.
+// the call's pairs spread over, for the choice of kernels.  With `phase`, the
+// pairs of the experts that the slots hold in it.
 int mfma_pairs(const void* x, int T, int H, int I, int K, const int32_t* slots, int nslots,
                const void* w13, size_t w13_stride, const void* w2, size_t w2_stride, void* act,
                void* work, size_t work_bytes, int spread, hipStream_t st,
-               const StageEvents* ev) {
+               const StageEvents* ev, const Phase* phase = nullptr) {
   if (!mfma_supported(H, I)) {
     wisp_set_last_error("MFMA path needs hidden and intermediate sizes that are multiples of 256",
                         "MFMA experts");
@@ -871,7 +898,11 @@ int mfma_pairs(const void* x, int T, int H, int I, int K, const int32_t* slots, 
   int32_t* lists = (int32_t*)((char*)work + W.lists);
   int32_t* counts = (int32_t*)((char*)work + W.counts);
   float* y = (float*)((char*)work + W.y);
-  launch_gather(slots, P, nslots, lists, counts, st);
+  if (phase)
+    gather(slots, P, nslots, lists, counts,
+           ((uintptr_t)slots | (uintptr_t)phase->ids) % 16 == 0, *phase, st);
+  else
+    launch_gather(slots, P, nslots, lists, counts, st);
   // A slot holds a token at most once (a token's top-k experts are
   // distinct), so T bounds the rows of any slot.
   const uint16_t* xb = (const uint16_t*)x;
@@ -898,18 +929,6 @@ int mfma_pairs(const void* x, int T, int H, int I, int K, const int32_t* slots, 
   return WISP_OK;
 }
 
-// slots[p] of one phase (see experts_mfma_phase).
-__global__ __launch_bounds__(256) void phase_slots_kernel(const int32_t* __restrict__ ids,
-                                                          const int32_t* __restrict__ slots,
-                                                          int P, PhaseTable t,
-                                                          int32_t* __restrict__ out) {
-  const int p = blockIdx.x * 256 + threadIdx.x;
-  if (p >= P) return;
-  const int e = ids[p];
-  const int s = e >= 0 && e < kMaxExperts ? t.slot[e] : PhaseTable::kNone;
-  out[p] = s == PhaseTable::kDecided ? slots[p] : s;
-}
-
 }  // namespace
 
 int experts_mfma(const void* x, int T, int H, int I, int K, const float* topk_w,
@@ -924,16 +943,15 @@ int experts_mfma(const void* x, int T, int H, int I, int K, const float* topk_w,
 }
 
 // The pairs of the experts that a phase of a paged call covers: their y rows
-// in the work buffer.  phase_slots: P ints of scratch.
+// in the work buffer.
 int experts_mfma_phase(const void* x, int T, int H, int I, int K, const int32_t* ids,
-                       const int32_t* slots, const PhaseTable& t, int32_t* phase_slots,
-                       int nslots, int num_experts, const void* w13, size_t w13_stride,
-                       const void* w2, size_t w2_stride, void* act, void* work,
-                       size_t work_bytes, hipStream_t st, const StageEvents* ev) {
-  hipLaunchKernelGGL(phase_slots_kernel, dim3((T * K + 255) / 256), dim3(256), 0, st, ids, slots,
-                     T * K, t, phase_slots);
-  return mfma_pairs(x, T, H, I, K, phase_slots, nslots, w13, w13_stride, w2, w2_stride, act, work,
-                    work_bytes, num_experts, st, ev);
+                       const int32_t* slots, const PhaseTable& t, int nslots, int num_experts,
+                       const void* w13, size_t w13_stride, const void* w2, size_t w2_stride,
+                       void* act, void* work, size_t work_bytes, hipStream_t st,
+                       const StageEvents* ev) {
+  const Phase phase{ids, t};
+  return mfma_pairs(x, T, H, I, K, slots, nslots, w13, w13_stride, w2, w2_stride, act, work,
+                    work_bytes, num_experts, st, ev, &phase);
 }
 
 // out from the y rows of every pair with a slot.

@@ -100,10 +100,10 @@ int experts_mfma(const void* x, int T, int H, int I, int K, const float* topk_w,
                  size_t work_bytes, hipStream_t st, const StageEvents* ev);
 size_t mfma_work_bytes(int T, int K, int H, int nslots);
 int experts_mfma_phase(const void* x, int T, int H, int I, int K, const int32_t* ids,
-                       const int32_t* slots, const PhaseTable& t, int32_t* phase_slots,
-                       int nslots, int num_experts, const void* w13, size_t w13_stride,
-                       const void* w2, size_t w2_stride, void* act, void* work,
-                       size_t work_bytes, hipStream_t st, const StageEvents* ev);
+                       const int32_t* slots, const PhaseTable& t, int nslots, int num_experts,
+                       const void* w13, size_t w13_stride, const void* w2, size_t w2_stride,
+                       void* act, void* work, size_t work_bytes, hipStream_t st,
+                       const StageEvents* ev);
 int experts_mfma_combine(int T, int H, int K, const float* topk_w, const int32_t* slots,
                          int nslots, const void* work, void* out, hipStream_t st);
 size_t fp8_work_bytes(int T, int K, int H, int I, int nslots);
@@ -730,11 +730,10 @@ int run_phases(Layer& L, const PhasePlan& plan, int T, int K, const void* x, voi
     if (p13 && p2) L.prof_w13_calls += 1;
     const StageEvents ev = {{p13 ? p13->start : nullptr, p13 ? p13->stop : nullptr,
                              p2 ? p2->start : nullptr, p2 ? p2->stop : nullptr}};
-    // ws->loads has served the pager and holds more than T * K words
-    failed = experts_mfma_phase(x, T, d.hidden, d.inter, K, ws->topk_ids, ws->slots, t, ws->loads,
-                                d.cap, d.num_experts, d.scratch_w13, d.scratch_w13_stride,
-                                d.scratch_w2, d.scratch_w2_stride, ws->act, ws->work,
-                                ws->work_bytes, st, (p13 && p2) ? &ev : nullptr);
+    failed = experts_mfma_phase(x, T, d.hidden, d.inter, K, ws->topk_ids, ws->slots, t, d.cap,
+                                d.num_experts, d.scratch_w13, d.scratch_w13_stride, d.scratch_w2,
+                                d.scratch_w2_stride, ws->act, ws->work, ws->work_bytes, st,
+                                (p13 && p2) ? &ev : nullptr);
     if (failed != WISP_OK) return;
     if (p13 && p2) p13->pending = p2->pending = true;
     if (hipEventRecord(L.ev_gemm[phase % kEventRing], st) == hipSuccess)
@@ -750,14 +749,14 @@ int run_phases(Layer& L, const PhasePlan& plan, int T, int K, const void* x, voi
     PageInList list;
     std::vector<int32_t> host(2 * ph.size());
     PhaseTable t;
-    for (int e = 0; e < kMaxExperts; ++e) t.slot[e] = PhaseTable::kNone;
+    for (int s = 0; s < kMaxExperts; ++s) t.expert[s] = PhaseTable::kNone;
     bool use = false;
     for (size_t j = 0; j < ph.size(); ++j) {
       list.pair[j][0] = ph[j].expert;
       list.pair[j][1] = ph[j].slot;
       host[2 * j] = ph[j].expert;
       host[2 * j + 1] = ph[j].slot;
-      if (ph[j].use) t.slot[ph[j].expert] = ph[j].slot;
+      if (ph[j].use) t.expert[ph[j].slot] = ph[j].expert;
       use = use || ph[j].use;
     }
     const int rc = L.kpin ? page_in_kernel(L, nullptr, nullptr, (int)ph.size(), st, nullptr, &list)
@@ -1310,7 +1309,7 @@ extern "C" int wisp_plan_phases(const int32_t* record, int T, int K, int E, int 
     return WISP_ERR_INVALID;
   const PhasePlan p = plan_phases(record, T, K, E, cap);
   if (p.loads > max_loads) return WISP_ERR_INVALID;
-  for (int e = 0; e < E; ++e) first[e] = p.first.slot[e];
+  for (int e = 0; e < E; ++e) first[e] = p.place[e];
   int n = 0;
   for (size_t i = 0; i < p.phases.size(); ++i)
     for (const PhaseLoad& l : p.phases[i]) {

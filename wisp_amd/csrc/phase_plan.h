@@ -33,6 +33,9 @@ struct PhaseLoad {
 
 struct PhasePlan {
   PhaseTable first;  // phase 0
+  // where phase 0 finds each expert: its slot before the call, kDecided for
+  // the slot that the pager decided, kNone where a later phase has it
+  std::vector<int16_t> place;
   std::vector<std::vector<PhaseLoad>> phases;
   int loads = 0;     // copies of the plan
   int recorded = 0;  // copies of the decision record
@@ -62,11 +65,14 @@ inline PhasePlan plan_phases(const int32_t* rec, int T, int K, int E, int cap) {
       ++p.recorded;
     }
   }
-  for (int e = 0; e < kMaxExperts; ++e)
-    p.first.slot[e] = e >= E           ? PhaseTable::kNone
-                      : home[e] >= 0   ? (int16_t)home[e]
-                      : loaded[e]      ? PhaseTable::kNone
-                                       : PhaseTable::kDecided;
+  for (int s = 0; s < kMaxExperts; ++s)
+    p.first.expert[s] = s < cap && !touched[s] ? PhaseTable::kDecided : PhaseTable::kNone;
+  for (int e = 0; e < E; ++e) {
+    if (home[e] >= 0) p.first.expert[home[e]] = (int16_t)e;
+    p.place.push_back(home[e] >= 0 ? (int16_t)home[e]
+                      : loaded[e]  ? PhaseTable::kNone
+                                   : PhaseTable::kDecided);
+  }
   // slots whose old expert is also their last keep it throughout, unless no
   // other slot is there for the experts that come and go
   std::vector<PhaseLoad> finals, kept;
