@@ -78,7 +78,8 @@ int wisp_record_words(int T, int K);
  * phase 0 finds expert e's weights (its slot before the call; -2: the slot
  * the pager decided; -1: a later phase has it); loads: one row of four words
  * per copy, {phase, expert, slot, 1 if that phase multiplies the expert's
- * tokens}.  Returns the number of copies, or WISP_ERR_INVALID. */
+ * tokens}.  Returns the number of copies, or -1 for invalid arguments (among
+ * them max_loads below that number). */
 int wisp_plan_phases(const int32_t* record, int T, int K, int E, int cap, int32_t* first,
                      int32_t* loads, int max_loads);
 

@@ -149,3 +149,27 @@ def test_phase_plan_serves_every_pair_and_leaves_the_decided_slots(hiplib, E, K,
         full = hp.s2e >= 0
         assert np.array_equal(held[full], hp.s2e[full]), step
     assert saved > 0 or cap == E - 1
+
+
+def test_phase_plan_of_one_copy_is_not_an_error(hiplib):
+    """Two tokens, one expert each, one empty slot that takes the second:
+    one copy.  The same call with no room for it, or without a record, is
+    refused with another value."""
+    hp = HostPager(4, 2)
+    hp.call([[0]])
+    ids = np.array([[0], [1]], dtype=np.int32)
+    words = hiplib.wisp_record_words(2, 1)
+    rec = np.zeros(words, dtype=np.int32)
+    slots = np.zeros(2, dtype=np.int32)
+    assert hiplib.wisp_pager_decide_host(
+        ids.ctypes.data, 2, 1, 4, 2, 0, hp.map.ctypes.data, hp.s2e.ctypes.data,
+        hp.tick.ctypes.data, hp.ctr.ctypes.data, slots.ctypes.data, rec.ctypes.data, words) == 0
+    first = np.zeros(4, dtype=np.int32)
+    loads = np.zeros((4, 4), dtype=np.int32)
+
+    def plan(record, most):
+        return hiplib.wisp_plan_phases(record, 2, 1, 4, 2, first.ctypes.data, loads.ctypes.data,
+                                       most)
+
+    assert plan(rec.ctypes.data, 4) == 1 and loads[0, 1] == 1
+    assert plan(rec.ctypes.data, 0) == -1 and plan(None, 4) == -1

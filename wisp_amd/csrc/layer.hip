@@ -1306,9 +1306,9 @@ extern "C" int wisp_plan_phases(const int32_t* record, int T, int K, int E, int 
   using namespace wisp;
   if (!record || T < 1 || K < 1 || E < 1 || E > kMaxExperts || cap < 1 || cap > kMaxExperts ||
       !first || (max_loads > 0 && !loads))
-    return WISP_ERR_INVALID;
+    return -1;
   const PhasePlan p = plan_phases(record, T, K, E, cap);
-  if (p.loads > max_loads) return WISP_ERR_INVALID;
+  if (p.loads > max_loads) return -1;
   for (int e = 0; e < E; ++e) first[e] = p.place[e];
   int n = 0;
   for (size_t i = 0; i < p.phases.size(); ++i)
