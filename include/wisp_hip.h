@@ -79,7 +79,7 @@ int wisp_record_words(int T, int K);
  * the pager decided; -1: a later phase has it); loads: one row of four words
  * per copy, {phase, expert, slot, 1 if that phase multiplies the expert's
  * tokens}.  Returns the number of copies, or -1 for invalid arguments (among
- * them max_loads below that number). */
+ * them max_loads below that number and a record word out of range). */
 int wisp_plan_phases(const int32_t* record, int T, int K, int E, int cap, int32_t* first,
                      int32_t* loads, int max_loads);
 

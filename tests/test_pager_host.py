@@ -173,3 +173,38 @@ def test_phase_plan_of_one_copy_is_not_an_error(hiplib):
 
     assert plan(rec.ctypes.data, 4) == 1 and loads[0, 1] == 1
     assert plan(rec.ctypes.data, 0) == -1 and plan(None, 4) == -1
+
+
+def test_phase_plan_refuses_a_damaged_record(hiplib):
+    """A word of the record that names no expert, slot, pair or group is
+    refused instead of followed."""
+    E, K, cap, T = 8, 2, 2, 6
+    hp = HostPager(E, cap)
+    rng = np.random.default_rng(3)
+    ids = np.stack([rng.choice(E, K, replace=False) for _ in range(T)]).astype(np.int32)
+    words = hiplib.wisp_record_words(T, K)
+    rec = np.zeros(words, dtype=np.int32)
+    slots = np.zeros(T * K, dtype=np.int32)
+    assert hiplib.wisp_pager_decide_host(
+        ids.ctypes.data, T, K, E, cap, 0, hp.map.ctypes.data, hp.s2e.ctypes.data,
+        hp.tick.ctypes.data, hp.ctr.ctypes.data, slots.ctypes.data, rec.ctypes.data, words) == 0
+    first = np.zeros(E, dtype=np.int32)
+    loads = np.zeros((T * K + E, 4), dtype=np.int32)
+
+    def plan(r):
+        return hiplib.wisp_plan_phases(r.ctypes.data, T, K, E, cap, first.ctypes.data,
+                                       loads.ctypes.data, len(loads))
+
+    assert plan(rec) > 0
+    evicted, loaded = 8 + 8 * T, 8 + 8 * T + 2 * T * K
+    group = 8 + 8 * (int(rec[1]) - 1)
+    assert rec[1] > 1 and rec[5] > 0 and rec[6] > 0
+    damage = [(1, T + 1), (1, -1), (evicted, E), (evicted, -1), (evicted + 1, cap),
+              (loaded, 1 << 20), (loaded, -7), (loaded + 1, cap), (loaded + 1, -1),
+              (group + 4, T * K + 1), (group + 5, T * K + 1), (group + 6, -1), (group + 7, -1),
+              (group + 7, 2 ** 31 - 1)]
+    for at, value in damage:
+        bad = rec.copy()
+        bad[at] = value
+        assert plan(bad) == -1, (at, value)
+    assert plan(rec) > 0

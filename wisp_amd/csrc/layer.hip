@@ -742,16 +742,16 @@ int run_phases(Layer& L, const PhasePlan& plan, int T, int K, const void* x, voi
       failed = WISP_ERR_HIP;
   };
   pairs(plan.first, 0);
-  const int n = (int)plan.phases.size();
-  for (int i = 0; i < n; ++i) {
-    const std::vector<PhaseLoad>& ph = plan.phases[i];
-    if (ph.empty() || (failed != WISP_OK && i + 1 < n)) continue;
+  for (int i = 0; i < plan.nphases; ++i) {
+    const PhaseLoad* ph = plan.load + plan.start[i];
+    const int n = plan.start[i + 1] - plan.start[i];
+    if (n == 0 || (failed != WISP_OK && i + 1 < plan.nphases)) continue;
     PageInList list;
-    std::vector<int32_t> host(2 * ph.size());
+    int32_t host[2 * kMaxExperts];
     PhaseTable t;
     for (int s = 0; s < kMaxExperts; ++s) t.expert[s] = PhaseTable::kNone;
     bool use = false;
-    for (size_t j = 0; j < ph.size(); ++j) {
+    for (int j = 0; j < n; ++j) {
       list.pair[j][0] = ph[j].expert;
       list.pair[j][1] = ph[j].slot;
       host[2 * j] = ph[j].expert;
@@ -759,8 +759,8 @@ int run_phases(Layer& L, const PhasePlan& plan, int T, int K, const void* x, voi
       if (ph[j].use) t.expert[ph[j].slot] = ph[j].expert;
       use = use || ph[j].use;
     }
-    const int rc = L.kpin ? page_in_kernel(L, nullptr, nullptr, (int)ph.size(), st, nullptr, &list)
-                          : page_in(L, host.data(), (int)ph.size(),
+    const int rc = L.kpin ? page_in_kernel(L, nullptr, nullptr, n, st, nullptr, &list)
+                          : page_in(L, host, n,
                                     last_gemm >= 0 ? L.ev_gemm[last_gemm % kEventRing] : nullptr,
                                     i, st);
     if (rc != WISP_OK) {
@@ -1173,8 +1173,9 @@ extern "C" int wisp_layer_forward(void* handle, const void* x, const void* logit
       rec[kRecGroupsDone] > 1) {
     // by phases when that copies less (a call whose groups load no expert
     // twice gains nothing from it)
-    const PhasePlan plan = plan_phases(rec, T, K, d.num_experts, d.cap);
-    if (plan.loads < plan.recorded) return run_phases(*L, plan, T, K, x, out, ws, st);
+    PhasePlan plan;
+    if (plan_phases(rec, T, K, d.num_experts, d.cap, &plan) && plan.loads < plan.recorded)
+      return run_phases(*L, plan, T, K, x, out, ws, st);
   }
   rc = run_groups(*L, rec, ws->loads, T, K, rec[kRecGroupsDone], status == WISP_OK, x,
                   ws->topk_w, ws->slots, ws->act, out, a, ws, st);
@@ -1307,16 +1308,19 @@ extern "C" int wisp_plan_phases(const int32_t* record, int T, int K, int E, int 
   if (!record || T < 1 || K < 1 || E < 1 || E > kMaxExperts || cap < 1 || cap > kMaxExperts ||
       !first || (max_loads > 0 && !loads))
     return -1;
-  const PhasePlan p = plan_phases(record, T, K, E, cap);
+  PhasePlan p;
+  if (!plan_phases(record, T, K, E, cap, &p)) {
+    wisp_set_last_error("decision record holds an out-of-range word", "wisp_plan_phases");
+    return -1;
+  }
   if (p.loads > max_loads) return -1;
   for (int e = 0; e < E; ++e) first[e] = p.place[e];
-  int n = 0;
-  for (size_t i = 0; i < p.phases.size(); ++i)
-    for (const PhaseLoad& l : p.phases[i]) {
-      const int32_t row[4] = {(int32_t)i, l.expert, l.slot, l.use};
-      memcpy(loads + 4 * n++, row, sizeof(row));
+  for (int i = 0; i < p.nphases; ++i)
+    for (int j = p.start[i]; j < p.start[i + 1]; ++j) {
+      const int32_t row[4] = {i, p.load[j].expert, p.load[j].slot, p.load[j].use};
+      memcpy(loads + 4 * j, row, sizeof(row));
     }
-  return n;
+  return p.loads;
 }
 
 extern "C" int wisp_layer_sync_record(void* handle, const wisp_workspace* ws) {
