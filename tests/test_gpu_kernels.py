@@ -292,11 +292,13 @@ def test_experts_gemv_bf16(T, H, I, E, K):
 # Calls of two or more tokens and at most 128 pairs read an expert's w13 rows
 # once for all of its pairs: pair counts around the 64 lanes of a wave and at
 # the limit and one over it, one expert for all, a pair without a slot.  The
-# longer I (129 and 130 chunks of 16 bytes) also share their w2 rows.
+# longer I (129 and 130 chunks of 16 bytes) also share their w2 rows, at H
+# 4096 for every call, at 2056 and 2048 from 24 pairs on.
 @pytest.mark.parametrize("T,K,E", [(2, 1, 1), (8, 8, 16), (13, 5, 9), (16, 8, 24), (43, 3, 7),
                                     (64, 2, 2)])
 @pytest.mark.parametrize("dtype,H,I", [(torch.bfloat16, 2048, 70), (torch.float32, 320, 33),
-                                       (torch.bfloat16, 264, 1032), (torch.float32, 132, 520)])
+                                       (torch.bfloat16, 4096, 1032),
+                                       (torch.bfloat16, 2056, 1032), (torch.float32, 2048, 520)])
 def test_gemv_bytes_with_shared_experts(T, K, E, dtype, H, I):
     I = I // 8 * 8
     x, w, ids, w13, w2 = _expert_case(T * 7 + K, T, H, I, E, K, dtype)

@@ -1145,9 +1145,17 @@ int dispatch_w2(const T* act, int T_, int H, int I, int K, const float* w, const
       case 3: launch_w2<T, 32, 3, 2>(act, T_, H, I, K, w, slots, w2, w2_stride, out, st, c); break;
       default: launch_w2<T, 32, 4, 2>(act, T_, H, I, K, w, slots, w2, w2_stride, out, st, c); break;
     }
-  } else if (T_ >= 2 && T_ * K <= kSharedPairs && !c.skip_if) {
-    // (not the shorter rows: layers of many small experts, whose tokens share
-    // few of them below the grouped GEMM's token counts)
+  } else if (T_ >= 2 && T_ * K <= kSharedPairs && !c.skip_if &&
+             (H >= 4096 || (H >= 2048 && T_ * K >= 24))) {
+    // From 4096 rows on its blocks fill the GPU and it is the faster one for
+    // every call; with 2048 it needs the sharing of 24 pairs; with fewer the
+    // per-pair blocks stay.  Measured, per pair against shared (us per call):
+    // 4096 x 1536, 64 experts top-4, 2 tokens 55.1 / 53.4; 4096 x 14336, 8
+    // top-2, 2 tokens 200 / 182; 2048 x 1536, 32 top-4, 4 / 6 / 13 tokens (16 /
+    // 24 / 52 pairs) 45.4 / 59.6 / 101 against 47.3 / 59.2 / 91; 1024 x 1536, 16
+    // top-2, 4 / 8 / 13 tokens 16.1 / 26.3 / 31.2 against 19.4 / 30.8 / 36.0.
+    // (Not the shorter rows: layers of many small experts, whose tokens share
+    // few of them below the grouped GEMM's token counts.)
     constexpr int RPH = 4;
     launch_timed(w2_shared_kernel<T, RPH>, dim3((H + RPH - 1) / RPH), dim3(64 * kSharedWaves), st,
                  c.start, c.stop, act, H, I, K, T_ * K, w, slots, w2, w2_stride, out, c.nslots);
