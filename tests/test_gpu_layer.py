@@ -764,3 +764,31 @@ def test_calls_by_phases_keep_the_loaded_pairs(monkeypatch, engine, streams, K, 
         # some expert is loaded again, so the call goes by phases
         assert len({e for e, _ in pairs}) < len(pairs) <= T * K
         assert st._ws.loads[:2 * len(pairs)].view(-1, 2).tolist() == pairs
+
+
+@pytest.mark.parametrize("T,K", [(1001, 5), (2051, 2)])
+def test_wide_calls_write_every_pairs_word(T, K):
+    """A call of more than 4096 pairs in one group, a count that no quad (and
+    with K 2 no pass of the block) divides: every pair's word holds its slot
+    and, where the call loaded the pair's expert, that expert + 1."""
+    H, I, E = 256, 256, 64
+    g = torch.Generator().manual_seed(T)
+    w13 = (torch.randn((E, 2 * I, H), generator=g) * 0.05).to(torch.bfloat16).pin_memory()
+    w2 = (torch.randn((E, H, I), generator=g) * 0.05).to(torch.bfloat16).pin_memory()
+    st = WispMoEState(w13, w2, E, "paged", DEV, 0)
+    for live in (50, E):  # the second call loads the last 14 experts
+        x = torch.randn((T, H), generator=g).to(torch.bfloat16).to(DEV)
+        lg = torch.randn((T, E), generator=g)
+        lg[:, live:] = -100.0
+        st.forward(x, lg.to(DEV), K, True)
+        torch.cuda.synchronize()
+        rec = parse_record(st.last_record.numpy(), T, K)
+        assert len(rec["groups"]) == 1
+        loaded = {e for e, _ in rec["groups"][0]["loaded"]}
+        assert loaded == set(range(50) if live == 50 else range(50, E))
+        ids = st.last_topk[1].reshape(-1).cpu()
+        slots = st.last_slots.reshape(-1).cpu()
+        new = torch.tensor([e in loaded for e in range(E)])[ids.long()]
+        want = slots + torch.where(new, (ids + 1) << 16, torch.zeros_like(ids))
+        assert int(st._ws.flags[0]) == len(loaded)
+        assert torch.equal(st._ws.flags[1:1 + T * K].cpu(), want)
