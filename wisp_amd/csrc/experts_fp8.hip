@@ -1570,7 +1570,9 @@ __global__ __launch_bounds__(256) void fp8_w2_dma_kernel(
 // instructions 190 + 125 us.  Measured and not better: issuing the next row
 // group's products before scaling this one's (302 + 156 us, registers spill),
 // 128 rows by 256 tokens (310 + 192), 256 by 128 tokens (290 + 165; 486 + 294
-// at 8192 tokens), sixteen waves (380 + 259, spills).
+// at 8192 tokens), sixteen waves (380 + 259, spills).  The kernels as they are
+// spill as well, outside the chunk loop (w13 11 registers, w2 3, stored and
+// read once a tile).
 // ---------------------------------------------------------------------------
 struct Fp8TileArgs {
   const uint8_t* A;      // codes: xq [T][H] (w13) or aq [P][I] (w2)
@@ -1790,6 +1792,7 @@ __global__ __launch_bounds__(64 * Sh::kWaves)
 __attribute__((amdgpu_waves_per_eu(Sh::kWaves / 4, Sh::kWaves / 4))) void fp8_tile_kernel(
     Fp8TileArgs a) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  static_assert(Sh::NT == 4, "token tiles of a wave in the dispatch below");
   tile::Table* tab = reinterpret_cast<tile::Table*>(smem + Sh::kTable);
   Fp8TileLoop<Sh, kW13> L{a, smem, tab};
   L.N = kW13 ? 2 * a.I : a.H;
@@ -1833,12 +1836,8 @@ __attribute__((amdgpu_waves_per_eu(Sh::kWaves / 4, Sh::kWaves / 4))) void fp8_ti
       L.template run<2>(w, src, p, &more);
     else if (nt == 3)
       L.template run<3>(w, src, p, &more);
-    else if (Sh::NT == 4 || nt == 4)
-      L.template run<4>(w, src, p, &more);
-    else if (nt == 5)
-      L.template run<(Sh::NT > 4 ? 5 : 4)>(w, src, p, &more);
     else
-      L.template run<(Sh::NT > 4 ? 6 : 4)>(w, src, p, &more);
+      L.template run<4>(w, src, p, &more);
   }
 }
 

@@ -803,7 +803,8 @@ hipError_t launch_tile(const TileArgs& a, hipStream_t st, hipEvent_t e0, hipEven
 // then tiles of 192, which split the larger slots.  Measured at the Mixtral
 // 1000-token chunk's w2 (8 slots of ~250 tokens, 16 panels): 392 against
 // 341 us; at the Qwen3 8192-token chunk (128 slots of ~512, 8 panels) 324
-// against 342 us, and its w13 466 against 509 us.
+// against 342 us, and its w13 466 against 509 us (before the halves of a w13
+// tile started apart).
 template <bool kW13>
 hipError_t launch_tiles(const TileArgs& a, hipStream_t st, hipEvent_t e0, hipEvent_t e1) {
   using Big = tile::Shape<2, 4, 8, 4>;

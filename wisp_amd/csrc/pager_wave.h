@@ -61,6 +61,16 @@ __device__ inline int set_table_size(int n) {
   return n <= 4 ? 8 : n <= 18 ? 32 : n <= 76 ? 128 : n <= 306 ? 512 : 2048;
 }
 
+// What the other waves of the pager's block do for a call whose ids do not
+// fit its LDS: before pager_wave they have read the ids (`bad`: one lies
+// outside [0, E); `all`: the experts they name), and after it they write the
+// slot and flag words of a call that is one group (`write`, set by
+// pager_wave).
+struct WideCall {
+  uint32_t all[kMaxExperts / 32];
+  int bad, write;
+};
+
 // One wavefront.  With `logits` non-null it first routes the T <= 8 tokens
 // (writing topk_w / topk_ids) and takes the ids from LDS; otherwise it reads
 // `ids_in` (staged in LDS when the call has at most kStagedPairs pairs).
@@ -100,16 +110,7 @@ __device__ inline int set_table_size(int n) {
 // REGS (decided at launch): a call whose ids were routed before the launch,
 // on the register path - batched decode and prefill chunks - compiled
 // without the routing and the LDS path.
-// What the other waves of the pager's block do for a call whose ids do not
-// fit its LDS: before pager_wave they have read the ids (`bad`: one lies
-// outside [0, E); `all`: the experts they name), and after it they write the
-// slot and flag words of a call that is one group (`write`, set by
-// pager_wave).
-struct WideCall {
-  uint32_t all[kMaxExperts / 32];
-  int bad, write;
-};
-
+// wide: the ids were read by the whole block (not staged).
 template <typename TL, int VALS, bool STAGED, int MAXE, int MAXP, bool ONE = false,
           bool REGS = false>
 __device__ __attribute__((always_inline)) inline void pager_wave(
