@@ -466,6 +466,22 @@ def test_w13_k_order_of_every_64_columns(H, I, E, per):
     assert (out.view(E, per, H) - (g * torch.sigmoid(g))[:, None]).abs().max() < 0.3
 
 
+# 256 MiB of y, where the sums start to read it non-temporally, and one token
+# less: a token's bytes are those of a call of its half of the tokens.
+@pytest.mark.parametrize("T", [4095, 4096])
+def test_mfma_sums_of_the_largest_calls(T):
+    H, I, E, K = 1024, 256, 32, 16
+    x, w, ids, w13, w2 = _expert_case(T, T, H, I, E, K, torch.bfloat16)
+    ids[T - 1, 3] = -1
+    xd, wd, idd, w13d, w2d = _dev_case(x, w, ids, w13, w2)
+    assert (T * K * H * 4 >= 256 << 20) == (T == 4096)
+    whole = run_experts(xd, wd, idd, w13d, w2d, algo=MFMA)
+    for a, b in [(0, T // 2), (T // 2, T)]:
+        part = run_experts(xd[a:b].contiguous(), wd[a:b].contiguous(), idd[a:b].contiguous(),
+                           w13d, w2d, algo=MFMA)
+        assert torch.equal(part.view(torch.int16), whole[a:b].view(torch.int16)), a
+
+
 def test_experts_mfma_absent_slot_contributes_zero():
     x, w, ids, w13, w2 = _expert_case(6, 20, 512, 256, 8, 2, torch.bfloat16)
     slots = torch.tensor(ids, dtype=torch.int32)

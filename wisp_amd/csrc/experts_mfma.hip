@@ -680,13 +680,17 @@ __attribute__((amdgpu_waves_per_eu(Sh::kWaves / 4, Sh::kWaves / 4))) void mfma_t
 // 4. combine: out[t, h] = bf16(sum_k w[t,k] * y[(t,k), h]), k ascending,
 // skipping pairs without a slot (their y rows are never written: selected
 // out, not multiplied by zero).  8 columns per thread, every k's slot,
-// weight and y loads issued before the sums; y is read once, non-temporally
-// (118 -> 100 us for the 537 MB of an 8192-token Qwen3 call).
+// weight and y loads issued before the sums.  A y of more than the last-level
+// cache is read non-temporally (kStream), a smaller one comes from that cache.
+// Measured at the Qwen3 shape, default against non-temporal loads (us): 9.1 /
+// 9.9 at 768 tokens (50 MB), 14.4 / 15.8 at 1024, 23.0 / 26.2 at 2048, 49.1 /
+// 49.9 at 4096 (268 MB), 119.5 / 99.0 at 8192.
 // grid = (ceil(H / 2048), T).
 // ---------------------------------------------------------------------------
 constexpr int kCombineK = 16;  // top-k handled with all loads up front; more loop
+constexpr size_t kCombineStream = 256ull << 20;  // bytes of y
 
-template <bool kVecStore>
+template <bool kVecStore, bool kStream>
 __global__ __launch_bounds__(256) void combine_kernel(const float* __restrict__ y, int H, int K,
                                                      int nslots, const float* __restrict__ topk_w,
                                                      const int32_t* __restrict__ slots,
@@ -708,8 +712,8 @@ __global__ __launch_bounds__(256) void combine_kernel(const float* __restrict__ 
         ok[k] = sl >= 0 && sl < nslots;
         w[k] = topk_w[p];
         const f32x4* yr = reinterpret_cast<const f32x4*>(y + (size_t)p * H + h);
-        lo[k] = __builtin_nontemporal_load(yr);
-        hi[k] = __builtin_nontemporal_load(yr + 1);
+        lo[k] = kStream ? __builtin_nontemporal_load(yr) : yr[0];
+        hi[k] = kStream ? __builtin_nontemporal_load(yr + 1) : yr[1];
       }
     }
 #pragma unroll
@@ -739,12 +743,14 @@ __global__ __launch_bounds__(256) void combine_kernel(const float* __restrict__ 
 void launch_combine(const float* y, int T, int H, int K, int nslots, const float* topk_w,
                     const int32_t* slots, uint16_t* out, hipStream_t st) {
   const dim3 grid((H + 2047) / 2048, T);
-  if (((uintptr_t)out | ((size_t)H * 2)) % 16 == 0)
-    hipLaunchKernelGGL(combine_kernel<true>, grid, dim3(256), 0, st, y, H, K, nslots, topk_w,
-                       slots, out);
+  auto go = [&](auto* kernel) {
+    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, st, y, H, K, nslots, topk_w, slots, out);
+  };
+  const bool vec = ((uintptr_t)out | ((size_t)H * 2)) % 16 == 0;
+  if ((size_t)T * K * H * 4 >= kCombineStream)
+    vec ? go(&combine_kernel<true, true>) : go(&combine_kernel<false, true>);
   else
-    hipLaunchKernelGGL(combine_kernel<false>, grid, dim3(256), 0, st, y, H, K, nslots, topk_w,
-                       slots, out);
+    vec ? go(&combine_kernel<true, false>) : go(&combine_kernel<false, false>);
 }
 
 template <int S2, int NG>
